@@ -190,11 +190,16 @@ LH_DEV uint32_t wave_append(uint32_t* counter, bool pred) {
     return base + lanes_below(m);
 }
 
-LH_DEV const MeshInfo& mesh_info_at(uint64_t addr) { return *reinterpret_cast<const MeshInfo*>(addr); }
+// The records' uint64 device addresses as pointers.  They go through the
+// global address space: a pointer made from an integer alone is generic, and
+// generic (flat) loads also count as LDS accesses and may return out of
+// order, so that the compiler waits for every load in flight, LDS or memory,
+// before it uses any one of them.
 template <class T>
 LH_DEV const T* ptr(uint64_t addr) {
-    return reinterpret_cast<const T*>(addr);
+    return (const T*)(reinterpret_cast<const __attribute__((address_space(1))) T*>(addr));
 }
+LH_DEV const MeshInfo& mesh_info_at(uint64_t addr) { return *ptr<MeshInfo>(addr); }
 
 LH_DEV uint64_t* sector(const lh_view& v, uint32_t pass) {
     return v.prefix_sums + size_t(pass) * (1 + v.instance_capacity);
@@ -203,7 +208,14 @@ LH_DEV uint64_t* sector(const lh_view& v, uint32_t pass) {
 // View sources: every kernel takes one of these and reads its view with
 // get(index).  OneView carries a single view by value (index ignored);
 // ViewTable reads entry `index` of a device-resident lh_view array, which is
-// how one launch covers every view of a batch with the same arithmetic.
+// how one launch covers every view of a batch with the same arithmetic.  The
+// table is written when the batch is made, so its entries are read through
+// the constant address space (scalar loads where the index is uniform), and
+// their pointers are marked as global ones (see ptr()).
+template <class T>
+LH_DEV T* global(T* p) {
+    return (T*)((__attribute__((address_space(1))) T*)p);
+}
 struct OneView {
     lh_view v;
     LH_HD uint32_t count() const { return 1; }
@@ -216,7 +228,20 @@ struct ViewTable {
     uint32_t* seg_offsets;        // [LH_NUM_PASSES * n + 1]
     const uint32_t* tile_offsets; // [n + 1] resolve tiles (8x8) per view, exclusive scan
     LH_HD uint32_t count() const { return n; }
-    LH_DEV const lh_view& get(uint32_t i) const { return views[i]; }
+    LH_DEV lh_view get(uint32_t i) const {
+        const auto* q = (const __attribute__((address_space(4))) lh_view*)(views + i);
+        lh_view v;
+        v.uniforms = global(q->uniforms), v.misc = global(q->misc), v.prefix_sums = global(q->prefix_sums);
+        v.draws = global(q->draws), v.counters = global(q->counters), v.visbuffer = global(q->visbuffer);
+        v.shadow_maps = global(q->shadow_maps), v.radiance = global(q->radiance), v.ldr = global(q->ldr);
+        v.scratch = global(static_cast<char*>(q->scratch)), v.scratch_bytes = q->scratch_bytes;
+        v.instance_capacity = q->instance_capacity, v.draw_capacity = q->draw_capacity;
+        v.width = q->width, v.height = q->height, v.shadow_size = q->shadow_size;
+        v.big_capacity = q->big_capacity, v.clip_capacity = q->clip_capacity, v.flags = q->flags;
+        v.history = global(q->history), v.tonemap_lut = global(q->tonemap_lut);
+        v.bin_capacity = q->bin_capacity, v.skybox_size = q->skybox_size, v.skybox = global(q->skybox);
+        return v;
+    }
 };
 
 }  // namespace lhd

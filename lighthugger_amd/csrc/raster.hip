@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(256) k_plan_segments(ViewTable vs, uint32_t pa
     __shared__ uint32_t cnt[LH_MAX_BATCH_SEGMENTS];
     const uint32_t nseg = vs.n * np;
     for (uint32_t k = threadIdx.x; k < nseg; k += blockDim.x) {
-        const lh_view& v = vs.views[k / np];
+        const lh_view& v = vs.get(k / np);
         cnt[k] = min(v.counters[LH_CNT_DRAWS + pass0 + k % np], v.draw_capacity);
     }
     __syncthreads();

@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(64) LH_WAVES_ATTR(4) k_resolve_batch(lh_scene 
         else
             hi = mid;
     }
-    const lh_view& v = vs.views[lo];
+    const lh_view& v = vs.get(lo);
     const uint32_t local = g - vs.tile_offsets[lo], tiles_x = (v.width + 7) / 8;
     resolve_tile(s, v, local % tiles_x, local / tiles_x, p);
 }
