@@ -325,14 +325,14 @@ lh_status lh_view_status(const lh_view* view, uint32_t* host_counters, lh_stream
  * reference, whose raster is fixed-function).  Results are independent of
  * them; the autotuner picks them per resolution class.  Process-global. */
 typedef struct lh_tuning {
-    uint32_t small_extent_px;  /* triangles whose vertex bbox fits in this many pixels (1..32) are
-                                  rasterized by one lane */
+    uint32_t small_extent_px;  /* tiled main-view raster: boxes of at most this many pixels a side
+                                  (1..32) are rasterized by one lane */
     uint32_t meshlet_blocks;   /* persistent grid of the per-meshlet raster (one wave per block) */
     uint32_t big_blocks;       /* persistent grid of the large-triangle raster */
     uint32_t clip_blocks;      /* persistent grid of the clipping kernel */
     uint32_t cull_blocks;      /* persistent grid of the meshlet cull */
-    uint32_t medium_extent_px; /* up to this extent (small_extent_px..64) the whole wave rasterizes
-                                  the triangle in place; larger ones go to the big-triangle queue */
+    uint32_t medium_extent_px; /* up to this extent (small_extent_px..64) a triangle is rasterized by
+                                  the wave that set it up; larger ones go to the big-triangle queue */
     uint32_t tile_item_entries; /* tiled main-view raster: binned meshlets per work item (8..512; 0 = 64) */
     uint32_t tile_blocks;       /* tiled main-view raster: persistent grid of 512-thread blocks (0 = 1024) */
     uint32_t tile_raster;       /* 1: the main view goes through the tiled raster (when its bin_capacity

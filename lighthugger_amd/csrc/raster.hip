@@ -19,14 +19,17 @@
 // One launch covers a pass set - the main view, or all four cascades - whose
 // draw lists are concatenated into one index space, so the persistent grid is
 // balanced across cascades of very different load.  Work split:
-//   k_raster_meshlets  one wave per surviving meshlet: its <= 64 vertices are
-//                      transformed once (one per lane) into LDS, then each lane
-//                      sets up <= 2 of its <= 124 triangles.  Triangles whose
-//                      vertex bbox fits in `small_extent` pixels are rasterized
-//                      in the lane with int32 edge functions; larger ones go to
-//                      the big queue, clip-crossing ones to the clip queue
-//                      (both appended with one atomic per wave, tagged with
-//                      the pass).
+//   k_raster_meshlets  one-wave blocks over the surviving meshlets: a wave
+//                      loads the heads of its next 64 draws together, requests
+//                      a meshlet's indices, corners and positions while the
+//                      one before is in hand, transforms its <= 64 vertices
+//                      (one per lane) into LDS and sets up its <= 124 triangles
+//                      (two per lane).  Triangles within `medium_extent` that
+//                      cover a pixel centre's row and column go to the wave's
+//                      triangle queue, rasterized 64 at a time (raster_queue);
+//                      larger ones go to the big queue, clip-crossing ones to
+//                      the clip queue (one atomic per wave, tagged with the
+//                      pass).  k_raster_alpha: the same for alpha-clip draws.
 //   k_raster_clip      clips queued triangles and queues the fan pieces.
 //   k_raster_big       queued triangles, one wave each (whole block for
 //                      boxes over kWaveBoxPx pixels).
@@ -37,14 +40,36 @@ using namespace lhr;
 
 namespace {
 
+// Occupancy target of the meshlet raster (waves per SIMD).  It is bound by
+// VALU issue (about 320 instructions a meshlet, most of them the transform and
+// the setup of triangles that cover nothing) and, before the heads and the
+// fetches were pipelined, by the chain of dependent loads.  Four cascades of
+// the 20,000-instance field (2.0 M meshlets), per launch: 1.99 ms with one
+// meshlet at a time and each round's few survivors in their own lanes; 2.06,
+// 1.53, 1.49, 1.48 ms at 8, 7, 6, 5 waves with the pipeline and the queue (at
+// 8 the 64 VGPRs spill); 1.41 ms with the spans of raster_queue.
+#ifndef LH_MESHLET_WAVES
+#define LH_MESHLET_WAVES 6
+#endif
+
+// Queues of the clip and large-triangle kernels.
+LH_DEV void queue_clip(const lh_view& v, uint32_t pass0, bool pred, uint32_t d, uint32_t t, uint32_t pi, bool alpha) {
+    if (ballot(pred) == 0) return;
+    const uint32_t slot = wave_append(&v.counters[LH_CNT_CLIP + pass0], pred);
+    if (!pred) return;
+    if (slot < v.clip_capacity)
+        queues(v).clip[slot] = make_uint2((d << LH_KEY_TRI_BITS) | t, pi | (alpha ? kClipAlpha : 0u));
+    else
+        atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
+}
+
 // ALPHA selects the draws of alpha-clip mesh infos (double-sided, alpha test
 // per sample); the opaque instantiation skips them.  The alpha instantiation
 // returns at once when the culls counted no alpha-clip draw in its passes.
 template <int KIND, class VS, bool ST, bool ALPHA>
-__global__ void __launch_bounds__(64) LH_RASTER_OCCUPANCY k_raster_meshlets(lh_scene s, VS vs, PassSet ps) {
-    __shared__ int32_t sX[64], sY[64];
-    __shared__ float sZ[64];
-    __shared__ uint32_t sO[64];
+LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) {
+    __shared__ WaveVerts wv;
+    __shared__ TriQueue queue;
     const uint32_t lane = threadIdx.x;
     if constexpr (ALPHA) {
         uint32_t n = 0;
@@ -53,131 +78,125 @@ __global__ void __launch_bounds__(64) LH_RASTER_OCCUPANCY k_raster_meshlets(lh_s
         if (wave_sum_u32(n) == 0) return;
     }
     const Segments<VS> seg(vs, ps);
-    const uint32_t total = seg.total();
-    Tally<ST> tally;
-    auto body = [&](uint32_t view, uint32_t pi, uint32_t d, bool clip_queued) {
-        const lh_view& v = vs.get(view);
-        const Pass p = make_pass(v, ps.pass0 + pi);
-        const Queues qs = queues(v);
-        uint32_t* clip_counter = &v.counters[LH_CNT_CLIP + ps.pass0];
-        uint32_t* big_counter = &v.counters[LH_CNT_BIG + ps.pass0];
-        const LhMat4 M = view_matrix<KIND>(v, p.pass);
-        const MeshletReference ref = p.draws[d];
-        const Instance& in = s.instances[ref.instance_index];
-        const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
-        if (((mi.flags & MESH_INFO_FLAGS_ALPHA_CLIP) != 0) != ALPHA) return;  // wave-uniform
-        const Meshlet& ml = ptr<Meshlet>(mi.meshlets)[ref.meshlet_index];
-        const uint32_t mid = s.instance_meshlet_base[ref.instance_index] + ref.meshlet_index;
-        const uint32_t nvert = ml.index_count, ntri = ml.triangle_count;
-        // both rounds' corner indices, issued before the vertex fetch so the
-        // two latencies overlap
-        const uint8_t* micro = ptr<uint8_t>(mi.micro_indices) + ml.triangle_offset;
-        uint32_t corners[2] = {0u, 0u};
-        for (uint32_t r = 0; r < 2; r++) {
-            const uint32_t t = lane + 64 * r;
-            if (t < ntri) corners[r] = uint32_t(micro[3 * t]) | (uint32_t(micro[3 * t + 1]) << 8) |
-                                       (uint32_t(micro[3 * t + 2]) << 16);
-        }
-        if (lane < nvert) {
-            f3 w = mat4_point(in.transform, load_position(mi, load_index(mi, ml.index_offset + lane)));
-            f4 c = mat4_mul_vec4(M, f4{w.x, w.y, w.z, 1.0f});
-            uint32_t oc = finite4(c) ? outcode(c) : kBadVertex;
-            // clipped and invalid vertices store zeros, so that the triangle
-            // setup below may read any corner
-            SV sv{0, 0, 0.0f};
-            if (oc == 0 && !project(c, p.W, p.H, sv)) oc = kBadVertex;
-            sX[lane] = sv.X;
-            sY[lane] = sv.Y;
-            sZ[lane] = sv.z;
-            sO[lane] = oc;
-        }
-        __syncthreads();
-        for (uint32_t round = 0; round < 2; round++) {
-            const uint32_t t = lane + 64 * round;
-            if (__ballot(t < ntri) == 0) break;
-            // Every lane sets up its triangle (lanes past the meshlet read
-            // corner 0 three times: zero area) and the class is computed
-            // without nested branches, whose exits would each re-zero the
-            // setup's registers.
-            const uint32_t packed = corners[round];
-            const uint32_t i0 = packed & 255u, i1 = (packed >> 8) & 255u, i2 = packed >> 16;
-            const uint32_t o0 = sO[i0], o1 = sO[i1], o2 = sO[i2];
-            SV v0{sX[i0], sY[i0], sZ[i0]}, v1{sX[i1], sY[i1], sZ[i1]}, v2{sX[i2], sY[i2], sZ[i2]};
-            int64_t area;
-            int32_t xlo, xhi, ylo, yhi, ex, ey;
-            const bool set = setup<KIND>(v0, v1, v2, p.W, p.H, area, xlo, xhi, ylo, yhi, ex, ey, ALPHA);
-            const bool drawn = t < ntri && ((o0 | o1 | o2) & kBadVertex) == 0 && (o0 & o1 & o2) == 0;
-            const int32_t e = max(ex, ey);
-            // 0 none, 1 clip queue (unless the tiled raster's binning queued
-            // it already), 2 big queue, 3 in-lane, 4 wave-cooperative
-            const uint32_t cls = !drawn                 ? 0u
-                                 : (o0 | o1 | o2) != 0  ? (clip_queued ? 0u : 1u)
-                                 : !set                 ? 0u
-                                 : e <= ps.small_extent ? 3u
-                                 : e <= ps.medium_extent ? 4u
-                                                         : 2u;
-            const uint32_t id = (mid << LH_KEY_TRI_BITS) | t;
-            uint32_t cslot = wave_append(clip_counter, cls == 1);
-            if (cls == 1) {
-                if (cslot < v.clip_capacity)
-                    qs.clip[cslot] = make_uint2((d << LH_KEY_TRI_BITS) | t, pi | (ALPHA ? kClipAlpha : 0u));
-                else
-                    atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
-            }
-            uint32_t bslot = wave_append(big_counter, cls == 2);
-            if (cls == 2) {
-                if (bslot < v.big_capacity)
-                    store_big(qs.big + bslot, v0, v1, v2, id, xlo, xhi, ylo, yhi, pi, ALPHA);
-                else
-                    atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
-            }
-            if (cls == 3)
-                raster_small<KIND, ST, ALPHA>(s, v, p, v0, v1, v2, int32_t(area), xlo, xhi, ylo, yhi, id, tally);
-            // Medium triangles: broadcast each lane's setup and raster it with the whole wave.
-            for (uint64_t med = ballot(cls == 4); med; med &= med - 1) {
-                const uint32_t l = first_lane(med);
-                const SV a{readlane(v0.X, l), readlane(v0.Y, l), readlane(v0.z, l)};
-                const SV b{readlane(v1.X, l), readlane(v1.Y, l), readlane(v1.z, l)};
-                const SV c{readlane(v2.X, l), readlane(v2.Y, l), readlane(v2.z, l)};
-                raster_wave<KIND, ST, ALPHA>(s, v, p, a, b, c, readlane(xlo, l), readlane(xhi, l), readlane(ylo, l),
-                                             readlane(yhi, l), (mid << LH_KEY_TRI_BITS) | (l + 64 * round), lane,
-                                             tally);
-            }
-        }
-        tally.flush(v, p.pass);
-        __syncthreads();
-    };
-    constexpr uint32_t C = Segments<VS>::kChunk;
-    if constexpr (C == 1) {
+    uint32_t total = seg.total();
+    const uint32_t* list = nullptr;
+    if constexpr (std::is_same<VS, OneView>::value) {
         if (ps.direct) {  // the draws the tiled raster left to this kernel
             const lh_view& v = vs.get(0);
             const lhs::ScratchLayout L = lhs::scratch_layout(v);
-            const uint32_t* list = reinterpret_cast<const uint32_t*>(static_cast<const char*>(v.scratch) + L.direct);
-            const uint32_t n = min(v.counters[LH_CNT_TILE_DIRECT], L.direct_capacity);
-            for (uint32_t k = blockIdx.x; k < n; k += gridDim.x) {
-                const uint32_t e = list[k];
-                uint32_t view, pi, d;
-                seg.find(e & ~lhs::kBinDirect, view, pi, d);
-                body(view, pi, d, (e & lhs::kBinDirect) != 0);
+            list = reinterpret_cast<const uint32_t*>(static_cast<const char*>(v.scratch) + L.direct);
+            total = min(v.counters[LH_CNT_TILE_DIRECT], L.direct_capacity);
+        }
+    }
+    Tally<ST> tally;
+    uint32_t held = 0;            // triangles in the queue
+    uint32_t at = ~0u;            // view << 3 | pass within the set that they belong to
+    Pass p{};
+    LhMat4 M{};
+    auto flush = [&]() {
+        if (held) raster_queue<KIND, ST, ALPHA>(s, M, p, queue, 0, held, lane, tally);
+        held = 0;
+        if (at != ~0u) tally.flush(vs.get(at >> 3), p.pass);
+    };
+    for (uint32_t k0 = 0;; k0 += 64) {
+        // the heads of the wave's next 64 draws, one per lane
+        const uint32_t g = seg.draw(k0 + lane);
+        const uint64_t some = ballot(g < total);
+        if (some == 0) break;
+        DrawHead head{};
+        uint32_t where = 0, draw = 0;
+        bool clip_queued = false;
+        if (g < total) {
+            const uint32_t e = list ? list[g] : g;
+            uint32_t view, pi;
+            seg.find(e & ~(list ? lhs::kBinDirect : 0u), view, pi, draw);
+            clip_queued = list && (e & lhs::kBinDirect) != 0;
+            where = view << 3 | pi;
+            const lh_view& v = vs.get(view);
+            head = load_head(s, v.draws[size_t(ps.pass0 + pi) * v.draw_capacity + draw]);
+        }
+        uint64_t todo = ballot(g < total && (((head.info >> 16) & MESH_INFO_FLAGS_ALPHA_CLIP) != 0) == ALPHA);
+        const uint64_t clip_done = ballot(clip_queued);
+        if (todo == 0) continue;
+        MeshletFetch next;
+        DrawHead h = head_of_lane(head, first_lane(todo));
+        next.request(h, lane);
+        next.request_position(h, lane);
+        while (todo) {
+            const uint32_t l = first_lane(todo);
+            todo &= todo - 1;
+            const DrawHead cur = h;
+            MeshletFetch f = next;
+            if (todo) {  // the next draw's indices and corners travel while this one is transformed
+                h = head_of_lane(head, first_lane(todo));
+                next.request(h, lane);
             }
-            return;
-        }
-        for (uint32_t g = blockIdx.x; g < total; g += gridDim.x) {
-            uint32_t view, pi, d;
-            seg.find(g, view, pi, d);
-            body(view, pi, d, false);
-        }
-    } else {
-        for (uint32_t c0 = blockIdx.x * C; c0 < total; c0 += gridDim.x * C) {
-            auto cur = seg.cursor(c0);
-            const uint32_t c1 = min(c0 + C, total);
-            for (uint32_t g = c0; g < c1; g++) {
-                uint32_t view, pi, d;
-                seg.at(cur, g, view, pi, d);
-                body(view, pi, d, false);
+            const uint32_t here = readlane_u32(where, l), d = readlane_u32(draw, l), pi = here & 7u;
+            const lh_view& v = vs.get(here >> 3);
+            if (here != at) {  // wave-uniform: another view or pass than the queue's
+                flush();
+                at = here;
+                p = make_pass(v, ps.pass0 + pi);
+                M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
+            }
+            const LhMat4 T = load_mat4(reinterpret_cast<uint64_t>(&s.instances[cur.instance].transform));
+            SV sv;
+            lds_order();
+            const bool clean = transform_vertices(cur, f, T, M, p.W, p.H, lane, wv, sv);
+            lds_order();
+            if (todo) next.request_position(h, lane);
+            const uint32_t ntri = cur.triangles();
+            for (uint32_t round = 0; round * 64 < ntri; round++) {
+                const uint32_t t = lane + 64 * round;
+                const TriSetup ts = triangle_setup<KIND>(wv, f.corners(cur, lane, round), t < ntri, clean, ALPHA, p.W, p.H);
+                if (!clean && !((clip_done >> l) & 1)) queue_clip(v, ps.pass0, ts.clip, d, t, pi, ALPHA);
+                const bool big = ts.inside && ts.extent > ps.medium_extent, push = ts.inside && !big;
+                const uint32_t id = (cur.mid << LH_KEY_TRI_BITS) | t;
+                if (ballot(big)) {
+                    const uint32_t slot = wave_append(&v.counters[LH_CNT_BIG + ps.pass0], big);
+                    if (big) {
+                        const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]},
+                            v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
+                        if (slot < v.big_capacity)
+                            store_big(queues(v).big + slot, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id, ts.xlo,
+                                      ts.xhi, ts.ylo, ts.yhi, pi, ALPHA);
+                        else
+                            atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
+                    }
+                }
+                const uint64_t pm = ballot(push);
+                if (pm == 0) continue;
+                if (push) {
+                    const uint32_t slot = held + lanes_below(pm);
+                    const int32_t X0 = ts.xlo * 256, Y0 = ts.ylo * 256;
+                    const uint32_t va = pack_xy(ts.a.x - X0, ts.a.y - Y0), vb = pack_xy(ts.b.x - X0, ts.b.y - Y0),
+                                   vc = pack_xy(ts.c.x - X0, ts.c.y - Y0);
+                    const uint32_t za = __float_as_uint(wv.Z[ts.i0]), zb = __float_as_uint(wv.Z[ts.i1]),
+                                   zc = __float_as_uint(wv.Z[ts.i2]);
+                    queue.box[slot] = make_uint4(uint32_t(ts.xlo) | uint32_t(ts.ylo) << 16, va, ts.swapped ? vc : vb,
+                                                 ts.swapped ? vb : vc);
+                    queue.att[slot] = make_uint4(za, ts.swapped ? zc : zb, ts.swapped ? zb : zc, id);
+                }
+                held += uint32_t(__popcll(pm));
+                if (held >= 64) {  // the last 64 entries: nothing moves
+                    held -= 64;
+                    raster_queue<KIND, ST, ALPHA>(s, M, p, queue, held, 64, lane, tally);
+                    lds_order();
+                }
             }
         }
     }
+    flush();
+}
+
+template <int KIND, class VS, bool ST>
+__global__ void __launch_bounds__(64) LH_WAVES_ATTR(LH_MESHLET_WAVES) k_raster_meshlets(lh_scene s, VS vs, PassSet ps) {
+    raster_meshlets<KIND, VS, ST, false>(s, vs, ps);
+}
+// The alpha test's texture fetch needs twice the registers.
+template <int KIND, class VS, bool ST>
+__global__ void __launch_bounds__(64) LH_WAVES_ATTR(4) k_raster_alpha(lh_scene s, VS vs, PassSet ps) {
+    raster_meshlets<KIND, VS, ST, true>(s, vs, ps);
 }
 
 // Clip polygon in homogeneous coordinates (Sutherland-Hodgman).
@@ -391,12 +410,12 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
     } else {
         mark(KIND == 0 ? "raster_meshlets_view" : "raster_meshlets_shadow", st);
     }
-    hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST, false>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs, ps);
+    hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs, ps);
     ps.direct = 0;
     const bool alpha = !(s.flags & LH_SCENE_OPAQUE_ONLY);
     if (alpha) {
         mark(KIND == 0 ? "raster_alpha_view" : "raster_alpha_shadow", st);
-        hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST, true>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs,
+        hipLaunchKernelGGL((k_raster_alpha<KIND, VS, ST>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs,
                            ps);
     }
     mark(KIND == 0 ? "raster_clip_view" : "raster_clip_shadow", st);
