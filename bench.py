@@ -544,7 +544,7 @@ def main():
     raster_atomics = {"fragments_per_pass": frags, "atomics_per_pass": atomics}
     for kind, lo, hi in (("view", 0, 1), ("shadow", 1, abi.NUM_PASSES)):
         kt = sum(per_frame.get(f"{k}_{kind}", 0.0)
-                 for k in ("raster_meshlets", "raster_clip", "raster_big", "tile_raster", "raster_direct"))
+                 for k in ("raster_meshlets", "raster_big", "tile_raster", "raster_direct"))
         if kt > 0:
             raster_atomics[f"{kind}_atomics_per_s_G"] = round(sum(atomics[lo:hi]) / (kt * 1e-3) / 1e9, 2)
     if not args.no_atomic_probe:

@@ -47,7 +47,8 @@ typedef void* lh_stream; /* hipStream_t */
 
 /* Device counters of one view (u32 each). */
 #define LH_CNT_DRAWS 0     /* + pass: surviving meshlets of the pass (may exceed draw_capacity) */
-#define LH_CNT_BIG 8       /* + pass: triangles queued for the large-triangle raster */
+#define LH_CNT_BIG 8       /* + pass: triangles queued for the large-triangle raster (the pieces of
+                              clipped triangles are rasterized without being queued) */
 #define LH_CNT_CLIP 16     /* + pass: triangles queued for clipping */
 #define LH_CNT_OVERFLOW 24 /* bit mask of LH_OVERFLOW_* */
 #define LH_CNT_FLAGS 25    /* bit mask of LH_FLAG_* */
@@ -329,7 +330,8 @@ typedef struct lh_tuning {
                                   (1..32) are rasterized by one lane */
     uint32_t meshlet_blocks;   /* persistent grid of the per-meshlet raster (one wave per block) */
     uint32_t big_blocks;       /* persistent grid of the large-triangle raster */
-    uint32_t clip_blocks;      /* persistent grid of the clipping kernel */
+    uint32_t clip_blocks;      /* no effect (must be non-zero): clip-crossing triangles run on the
+                                  large-triangle raster's grid */
     uint32_t cull_blocks;      /* persistent grid of the meshlet cull */
     uint32_t medium_extent_px; /* up to this extent (small_extent_px..64) a triangle is rasterized by
                                   the wave that set it up; larger ones go to the big-triangle queue */

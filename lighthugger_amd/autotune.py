@@ -26,7 +26,6 @@ SPACE = {
     "medium_extent_px": [8, 12, 16, 32, 64],
     "meshlet_blocks": [4096, 8192, 16384],
     "big_blocks": [512, 2048],
-    "clip_blocks": [64, 256],
     "cull_blocks": [512, 1024, 2048],
     "tile_item_entries": [32, 64, 128],
     "tile_blocks": [768, 1024, 2048],

@@ -58,12 +58,6 @@ LH_DEV const LhMat4& view_matrix(const lh_view& v, uint32_t pass) {
     return KIND == 0 ? v.uniforms->combined_perspective_view : v.misc->shadow_matrices[pass - 1];
 }
 
-// The alpha test of one covered sample (alpha-clip geometry only).
-template <int KIND>
-LH_DEV bool alpha_pass(const lh_scene& s, const lh_view& v, const Pass& p, uint32_t id, int32_t px, int32_t py) {
-    return shading::alpha_visible(s, view_matrix<KIND>(v, p.pass), p.W, p.H, id, px, py);
-}
-
 LH_DEV Pass make_pass(const lh_view& v, uint32_t pass) {
     Pass p;
     p.pass = pass;
@@ -195,22 +189,29 @@ struct Tally<true> {
     }
 };
 
-// Depth test of one covered sample; returns whether an atomic was issued.
-// The atomic is issued without reading the target first: a read-before-
-// atomic early-out saves atomics but makes every sample wait for a load,
-// and measured slower (the raster is latency-bound, not atomic-bound).
-template <int KIND>
-LH_DEV bool fragment(const Pass& p, int32_t px, int32_t py, float z, uint32_t id) {
+// Depth test of one covered sample that `visible()` (the alpha test) lets
+// pass.  Without EARLY the atomic is issued without reading the target first:
+// in the meshlet raster a read-before-atomic early-out saves atomics but makes
+// every sample wait for a load.  With EARLY the target is read first, and a
+// sample that loses against what it holds costs neither an alpha test nor an
+// atomic (the value read may be an old one, which is only larger).
+template <int KIND, bool ST, bool EARLY, class F>
+LH_DEV void fragment(const Pass& p, int32_t px, int32_t py, float z, uint32_t id, Tally<ST>& tally, F&& visible) {
     z = fminf(fmaxf(z, 0.0f), 1.0f);
-    size_t o = size_t(py) * p.W + uint32_t(px);
+    const size_t o = size_t(py) * p.W + uint32_t(px);
     if (KIND == 0) {
-        if (!(z > 0.0f)) return false;  // depth GREATER against the 0.0 clear
-        unsigned long long key = ((unsigned long long)(~__float_as_uint(z)) << 32) | id;
-        atomicMin(reinterpret_cast<unsigned long long*>(p.vis + o), key);
+        const bool issue = z > 0.0f;  // depth GREATER against the 0.0 clear
+        const unsigned long long key = ((unsigned long long)(~__float_as_uint(z)) << 32) | id;
+        if (EARLY && (!issue || key >= p.vis[o])) return;
+        if (!visible()) return;
+        tally.hit(issue);
+        if (issue) atomicMin(reinterpret_cast<unsigned long long*>(p.vis + o), key);
     } else {
+        if (EARLY && __float_as_uint(z) >= p.depth[o]) return;
+        if (!visible()) return;
+        tally.hit(true);
         atomicMin(p.depth + o, __float_as_uint(z));
     }
-    return true;
 }
 
 LH_DEV int32_t readlane(int32_t v, uint32_t l) { return __builtin_amdgcn_readlane(v, int(l)); }
@@ -395,7 +396,11 @@ struct TriSetup {
     uint32_t i0, i1, i2;
     bool clip, inside, swapped;  // inside: faces the right way, covers a pixel centre's row and column
 };
-constexpr int32_t kNarrow = 64 * 256;  // extents up to 64 px: products of differences fit 24 x 24 -> 28 bits
+// Extents (subpixels) up to which the edge functions are evaluated in 32 bits:
+// at 120 px a difference has 15 bits and a step 23, so that the 24-bit
+// multiplier is exact, and an edge value within two pixels of the box stays
+// below 2 x 30720 x 31232 < 2^31; the area stays below 2^30 (rcp_exact).
+constexpr int32_t kNarrow = 120 * 256;
 template <int KIND>
 LH_DEV TriSetup triangle_setup(const WaveVerts& wv, uint32_t corners, bool live, bool clean, bool two_sided, uint32_t W,
                                uint32_t H) {
@@ -417,7 +422,7 @@ LH_DEV TriSetup triangle_setup(const WaveVerts& wv, uint32_t corners, bool live,
     t.extent = max(maxX - minX, maxY - minY);
     t.clip = drawn && !whole;
     t.inside = drawn && whole && t.xlo <= t.xhi && t.ylo <= t.yhi;
-    // Sign of the area.  Within 64 px the products are exact on the 24-bit
+    // Sign of the area.  Within kNarrow the products are exact on the 24-bit
     // multiplier; only a wave with a larger triangle that may be drawn takes
     // the 64-bit ones.
     bool neg, pos;
@@ -433,21 +438,49 @@ LH_DEV TriSetup triangle_setup(const WaveVerts& wv, uint32_t corners, bool live,
     return t;
 }
 
-// Triangles of up to 64 px that are ready to be rasterized, collected over a
+// Triangles of up to kNarrow that are ready to be rasterized, collected over a
 // wave's meshlets.  Most set-up triangles of a dense scene cover no pixel
 // centre (4 of 64 do in the cascades of the 2,000-instance field), so the
 // survivors of many rounds are put together here and rasterized 64 at a time
 // instead of a few lanes per round.  An entry holds its box origin, the
-// snapped vertices relative to the origin's pixel corner (16 bits each:
-// within 64 px of it), the three depths and the key's id; triangles are
+// snapped vertices relative to the origin's pixel corner (16 bits each), the three depths and the key's id; triangles are
 // oriented to positive area.  A round adds at most 64 entries to at most 63.
 constexpr uint32_t kQueue = 128;
-struct TriQueue {
-    uint4 box[kQueue];  // xlo | ylo << 16, v0, v1, v2 (x & 0xFFFF | y << 16)
-    uint4 att[kQueue];  // z0, z1, z2, id
-    int32_t own[64];    // owners of a pass's runs
+template <uint32_t N>
+struct TriQueueOf {
+    uint4 box[N];     // xlo | ylo << 16, v0, v1, v2 (x & 0xFFFF | y << 16)
+    uint4 att[N];     // z0, z1, z2, id
+    int32_t own[64];  // owners of a pass's runs
+    // a triangle of positive area; (xlo, ylo): first pixel of its clamped box
+    LH_DEV void store(uint32_t k, int32_t xlo, int32_t ylo, const SV& v0, const SV& v1, const SV& v2, uint32_t id) {
+        auto rel = [&](const SV& v) {
+            return (uint32_t(v.X - xlo * 256) & 0xFFFFu) | uint32_t(v.Y - ylo * 256) << 16;
+        };
+        box[k] = make_uint4(uint32_t(xlo) | uint32_t(ylo) << 16, rel(v0), rel(v1), rel(v2));
+        att[k] = make_uint4(__float_as_uint(v0.z), __float_as_uint(v1.z), __float_as_uint(v2.z), id);
+    }
 };
-LH_DEV uint32_t pack_xy(int32_t x, int32_t y) { return (uint32_t(x) & 0xFFFFu) | uint32_t(y) << 16; }
+using TriQueue = TriQueueOf<kQueue>;
+
+// shading::AlphaTri of up to 64 triangles, in LDS.
+struct AlphaStore {
+    float4 a[64], b[64], c[64], d[64], e[64];
+    LH_DEV void store(uint32_t k, const shading::AlphaTri& t) {
+        a[k] = make_float4(t.bary.invW.x, t.bary.invW.y, t.bary.invW.z, t.bary.n0.x);
+        b[k] = make_float4(t.bary.n0.y, t.bary.ddx.x, t.bary.ddx.y, t.bary.ddx.z);
+        c[k] = make_float4(t.bary.ddy.x, t.bary.ddy.y, t.bary.ddy.z, __uint_as_float(t.texture));
+        d[k] = make_float4(t.uv[0].x, t.uv[0].y, t.uv[1].x, t.uv[1].y);
+        e[k] = make_float4(t.uv[2].x, t.uv[2].y, t.offset.x, t.offset.y);
+    }
+    LH_DEV shading::AlphaTri load(uint32_t k) const {
+        const float4 p = a[k], q = b[k], r = c[k], u = d[k], w = e[k];
+        return {{{p.x, p.y, p.z}, {p.w, q.x}, {q.y, q.z, q.w}, {r.x, r.y, r.z}},
+                {{u.x, u.y}, {u.z, u.w}, {w.x, w.y}},
+                {w.z, w.w},
+                __float_as_uint(r.w)};
+    }
+};
+struct NoAlpha {};
 LH_DEV int32_t lo16(uint32_t v) { return int32_t(int16_t(v & 0xFFFFu)); }
 LH_DEV int32_t hi16(uint32_t v) { return int32_t(v) >> 16; }
 
@@ -459,7 +492,8 @@ struct QueuedTri {
     uint32_t id;
     LH_DEV int32_t area() const { return __mul24(bx - ax, cy - ay) - __mul24(by - ay, cx - ax); }
 };
-LH_DEV QueuedTri load_tri(const TriQueue& q, uint32_t k, uint32_t W, uint32_t H) {
+template <class Q>
+LH_DEV QueuedTri load_tri(const Q& q, uint32_t k, uint32_t W, uint32_t H) {
     const uint4 b = q.box[k], t = q.att[k];
     QueuedTri r;
     r.xlo = int32_t(b.x & 0xFFFFu), r.ylo = int32_t(b.x >> 16);
@@ -474,7 +508,7 @@ LH_DEV QueuedTri load_tri(const TriQueue& q, uint32_t k, uint32_t W, uint32_t H)
 }
 
 // Edge functions of a queued triangle along one pixel row.  Every difference
-// is within 64 px, so the values are exact on the 24-bit multiplier and step
+// is within kNarrow, so the values are exact on the 24-bit multiplier and step
 // exactly in integers: E_i(Px + 256) = E_i(Px) - 256 (Yb - Ya).  A pixel
 // centre on an edge counts when the edge is a top or left one, so coverage
 // (E > 0 || (E == 0 && top-left)) is E >= m with m = top-left ? 0 : 1.
@@ -494,12 +528,12 @@ struct RowEdges {
 };
 // Narrows the covered columns [lo, hi] of a row by one edge, exactly: the
 // quotient's estimate is within 1e-4 of (m - e) / s for the columns in
-// question (0..64; others are clamped away), so the column it names or the
+// question (0..120; others are clamped away), so the column it names or the
 // next one inward is the edge's own, and one evaluation of the edge says which.
 LH_DEV void clip_row(int32_t e, int32_t s, int32_t m, int32_t& lo, int32_t& hi) {
     const float q = float(m - e) * __builtin_amdgcn_rcpf(float(s));
     const float guess = s > 0 ? ceilf(q - 0.001f) : floorf(q + 0.001f);
-    int32_t c = int32_t(fminf(fmaxf(guess, -1.0f), 65.0f));
+    int32_t c = int32_t(fminf(fmaxf(guess, -1.0f), 121.0f));
     const int32_t miss = e + __mul24(c, s) < m ? 1 : 0;
     if (s > 0)
         lo = max(lo, c + miss);
@@ -510,13 +544,12 @@ LH_DEV void clip_row(int32_t e, int32_t s, int32_t m, int32_t& lo, int32_t& hi) 
 }
 
 // Depth test of the pixel at (x, y) of a queued triangle's box.
-template <int KIND, bool ST, bool ALPHA>
-LH_DEV void raster_pixel(const lh_scene& s, const LhMat4& M, const Pass& p, const QueuedTri& t, float inv_area, int32_t e1,
-                         int32_t e2, int32_t x, int32_t y, Tally<ST>& tally) {
+template <int KIND, bool ST, bool EARLY, class F>
+LH_DEV void raster_pixel(const Pass& p, const QueuedTri& t, float inv_area, int32_t e1, int32_t e2, int32_t x, int32_t y,
+                         Tally<ST>& tally, F&& visible) {
     const int32_t px = t.xlo + x, py = t.ylo + y;
-    if (ALPHA && !shading::alpha_visible(s, M, p.W, p.H, t.id, px, py)) return;
     const float l1 = float(e1) * inv_area, l2 = float(e2) * inv_area;
-    tally.hit(fragment<KIND>(p, px, py, (t.z0 + l1 * t.d10) + l2 * t.d20, t.id));
+    fragment<KIND, ST, EARLY>(p, px, py, (t.z0 + l1 * t.d10) + l2 * t.d20, t.id, tally, [&] { return visible(px, py); });
 }
 
 // Numbers the `n` pieces of work of each lane in lane order and hands them out
@@ -548,27 +581,28 @@ LH_DEV void wave_spread(int32_t* own, uint32_t lane, uint32_t n, F&& f) {
 // per lane, each cut to the columns that the triangle covers (exactly, so no
 // pixel is tested again); then the rows' covered pixels in runs of up to four.
 // So the cost follows the covered pixels, not the boxes: a sliver across a
-// 64 px box costs its rows and the few pixels on each.  The alpha test is far
+// 120 px box costs its rows and the few pixels on each.  The alpha test is far
 // dearer than the coverage: its runs are single pixels.  Against boxes walked
 // in runs of four with the edges tested at each pixel: the main views of 12
 // cameras 2.77 -> 1.96 ms, the alpha-clipped 720p view 1.12 -> 0.56 ms.
 constexpr int32_t kLanePx = 4;
-template <int KIND, bool ST, bool ALPHA>
-LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, TriQueue& q, uint32_t from, uint32_t n,
+template <int KIND, bool ST, bool ALPHA, bool EARLY, class Q, class A>
+LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q, A& alpha, uint32_t from, uint32_t n,
                          uint32_t lane, Tally<ST>& tally) {
     lds_order();
-    constexpr int32_t run = ALPHA ? 1 : 4;
     uint32_t rows = 0;
     float inv_area = 0.0f;
     if (lane < n) {
         const QueuedTri t = load_tri(q, from + lane, p.W, p.H);
         inv_area = rcp_exact(float(t.area()));
+        if constexpr (ALPHA) alpha.store(lane, shading::alpha_setup(s, M, t.id));
         if (!ALPHA && __mul24(t.w, t.h) <= kLanePx) {
             for (int32_t y = 0; y < t.h; y++) {
                 RowEdges r(t, y);
                 for (int32_t x = 0; x < t.w; x++) {
                     if (r.e0 >= r.m0 && r.e1 >= r.m1 && r.e2 >= r.m2)
-                        raster_pixel<KIND, ST, ALPHA>(s, M, p, t, inv_area, r.e1, r.e2, x, y, tally);
+                        raster_pixel<KIND, ST, EARLY>(p, t, inv_area, r.e1, r.e2, x, y, tally,
+                                                      [](int32_t, int32_t) { return true; });
                     r.e0 += r.s0, r.e1 += r.s1, r.e2 += r.s2;
                 }
             }
@@ -577,7 +611,7 @@ LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, TriQ
         }
     }
     wave_spread(q.own, lane, rows, [&](int32_t o, uint32_t y, bool active) {
-        uint32_t runs = 0, row = 0;  // row: first column | y << 8 | columns << 16 | triangle << 24
+        uint32_t columns = 0, row = 0;  // row: first column | y << 8 | triangle << 16
         if (active) {
             const QueuedTri t = load_tri(q, from + uint32_t(o), p.W, p.H);
             const RowEdges r(t, int32_t(y));
@@ -585,26 +619,26 @@ LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, TriQ
             clip_row(r.e0, r.s0, r.m0, lo, hi);
             clip_row(r.e1, r.s1, r.m1, lo, hi);
             clip_row(r.e2, r.s2, r.m2, lo, hi);
-            const int32_t len = hi - lo + 1;
-            if (len > 0) {
-                runs = uint32_t(len + run - 1) / uint32_t(run);
-                row = uint32_t(lo) | y << 8 | uint32_t(len) << 16 | uint32_t(o) << 24;
+            if (hi >= lo) {
+                columns = uint32_t(hi - lo + 1);
+                row = uint32_t(lo) | y << 8 | uint32_t(o) << 16;
             }
         }
-        wave_spread(q.own, lane, runs, [&](int32_t ro, uint32_t k, bool on) {
+        wave_spread(q.own, lane, columns, [&](int32_t ro, uint32_t k, bool on) {
             const uint32_t rw = uint32_t(__shfl(int32_t(row), ro, 64));
-            const uint32_t to = rw >> 24;
+            const uint32_t to = rw >> 16;
             const float inv = __shfl(inv_area, int32_t(to), 64);
             if (on) {
                 const QueuedTri t = load_tri(q, from + to, p.W, p.H);
-                const int32_t ry = int32_t(rw >> 8 & 255u), x0 = int32_t(rw & 255u) + run * int32_t(k);
-                const int32_t len = min(run, int32_t(rw >> 16 & 255u) - run * int32_t(k));
+                const int32_t ry = int32_t(rw >> 8 & 255u), x = int32_t((rw & 255u) + k);
                 const RowEdges r(t, ry);
-                int32_t e1 = r.e1 + __mul24(x0, r.s1), e2 = r.e2 + __mul24(x0, r.s2);
-                for (int32_t j = 0; j < len; j++) {
-                    raster_pixel<KIND, ST, ALPHA>(s, M, p, t, inv, e1, e2, x0 + j, ry, tally);
-                    e1 += r.s1, e2 += r.s2;
-                }
+                raster_pixel<KIND, ST, EARLY>(p, t, inv, r.e1 + __mul24(x, r.s1), r.e2 + __mul24(x, r.s2), x, ry, tally,
+                                              [&](int32_t px, int32_t py) {
+                                                  if constexpr (ALPHA)
+                                                      return shading::alpha_at(s, alpha.load(to), p.W, p.H, px, py);
+                                                  else
+                                                      return true;
+                                              });
             }
         });
     });

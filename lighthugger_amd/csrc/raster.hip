@@ -30,9 +30,8 @@
 //                      larger ones go to the big queue, clip-crossing ones to
 //                      the clip queue (one atomic per wave, tagged with the
 //                      pass).  k_raster_alpha: the same for alpha-clip draws.
-//   k_raster_clip      clips queued triangles and queues the fan pieces.
-//   k_raster_big       queued triangles, one wave each (whole block for
-//                      boxes over kWaveBoxPx pixels).
+//   k_raster_big       the queued large triangles, up to 64 to a wave, and the
+//                      clip-crossing ones, one to a block.
 #include "raster.h"
 
 using namespace lhd;
@@ -70,6 +69,7 @@ template <int KIND, class VS, bool ST, bool ALPHA>
 LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) {
     __shared__ WaveVerts wv;
     __shared__ TriQueue queue;
+    __shared__ std::conditional_t<ALPHA, AlphaStore, NoAlpha> alpha;
     const uint32_t lane = threadIdx.x;
     if constexpr (ALPHA) {
         uint32_t n = 0;
@@ -89,12 +89,16 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
         }
     }
     Tally<ST> tally;
+    // The early test pays where it saves an alpha test (statistics count every
+    // covered sample and do without); without one it costs: the cascades of
+    // the 20,000-instance field 1.17 -> 1.25 ms.
+    constexpr bool kEarly = ALPHA && !ST;
     uint32_t held = 0;            // triangles in the queue
     uint32_t at = ~0u;            // view << 3 | pass within the set that they belong to
     Pass p{};
     LhMat4 M{};
     auto flush = [&]() {
-        if (held) raster_queue<KIND, ST, ALPHA>(s, M, p, queue, 0, held, lane, tally);
+        if (held) raster_queue<KIND, ST, ALPHA, kEarly>(s, M, p, queue, alpha, 0, held, lane, tally);
         held = 0;
         if (at != ~0u) tally.flush(vs.get(at >> 3), p.pass);
     };
@@ -167,20 +171,15 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
                 const uint64_t pm = ballot(push);
                 if (pm == 0) continue;
                 if (push) {
-                    const uint32_t slot = held + lanes_below(pm);
-                    const int32_t X0 = ts.xlo * 256, Y0 = ts.ylo * 256;
-                    const uint32_t va = pack_xy(ts.a.x - X0, ts.a.y - Y0), vb = pack_xy(ts.b.x - X0, ts.b.y - Y0),
-                                   vc = pack_xy(ts.c.x - X0, ts.c.y - Y0);
-                    const uint32_t za = __float_as_uint(wv.Z[ts.i0]), zb = __float_as_uint(wv.Z[ts.i1]),
-                                   zc = __float_as_uint(wv.Z[ts.i2]);
-                    queue.box[slot] = make_uint4(uint32_t(ts.xlo) | uint32_t(ts.ylo) << 16, va, ts.swapped ? vc : vb,
-                                                 ts.swapped ? vb : vc);
-                    queue.att[slot] = make_uint4(za, ts.swapped ? zc : zb, ts.swapped ? zb : zc, id);
+                    const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]},
+                        v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
+                    queue.store(held + lanes_below(pm), ts.xlo, ts.ylo, v0, ts.swapped ? v2 : v1,
+                                ts.swapped ? v1 : v2, id);
                 }
                 held += uint32_t(__popcll(pm));
                 if (held >= 64) {  // the last 64 entries: nothing moves
                     held -= 64;
-                    raster_queue<KIND, ST, ALPHA>(s, M, p, queue, held, 64, lane, tally);
+                    raster_queue<KIND, ST, ALPHA, kEarly>(s, M, p, queue, alpha, held, 64, lane, tally);
                     lds_order();
                 }
             }
@@ -204,162 +203,250 @@ LH_DEV f4 clip_point(f4 a, f4 b, float da, float db) {
     float t = da / (da - db);
     return {a.x + (b.x - a.x) * t, a.y + (b.y - a.y) * t, a.z + (b.z - a.z) * t, a.w + (b.w - a.w) * t};
 }
+// Alpha-clipped triangles over this extent go to the large-triangle raster,
+// which spreads them over the chip: their samples are far dearer than opaque
+// ones, and a wave would keep its meshlet's to itself (1,500 alpha-clipped
+// cards at 720p: 1.07, 0.88, 0.71, 0.68, 0.67 ms a frame at 16, 12, 8, 6, 4 px).
+constexpr int32_t kAlphaMediumPx = 6;
 
-// View blockIdx.z; grid-stride over that view's clip queue.
-template <int KIND, class VS>
-__global__ void __launch_bounds__(64) k_raster_clip(lh_scene s, VS vs, PassSet ps) {
-    const lh_view& v = vs.get(blockIdx.z);
-    const Queues qs = queues(v);
-    const uint32_t count = min(v.counters[LH_CNT_CLIP + ps.pass0], v.clip_capacity);
-    uint32_t* big_counter = &v.counters[LH_CNT_BIG + ps.pass0];
-    for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < count; q += gridDim.x * blockDim.x) {
-        const uint2 e = qs.clip[q];
-        const uint32_t d = e.x >> LH_KEY_TRI_BITS, t = e.x & ((1u << LH_KEY_TRI_BITS) - 1), pi = e.y & ~kClipAlpha;
-        const bool alpha = (e.y & kClipAlpha) != 0;
-        const Pass p = make_pass(v, ps.pass0 + pi);
-        const LhMat4 M = view_matrix<KIND>(v, p.pass);
-        const MeshletReference ref = p.draws[d];
-        const Instance& in = s.instances[ref.instance_index];
-        const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
-        const Meshlet& ml = ptr<Meshlet>(mi.meshlets)[ref.meshlet_index];
-        const uint32_t mid = s.instance_meshlet_base[ref.instance_index] + ref.meshlet_index;
-        const uint8_t* micro = ptr<uint8_t>(mi.micro_indices) + ml.triangle_offset;
-        f4 poly[12], tmp[12];
-        for (int j = 0; j < 3; j++) {
-            f3 w = mat4_point(in.transform, load_position(mi, load_index(mi, ml.index_offset + micro[3 * t + j])));
-            poly[j] = mat4_mul_vec4(M, f4{w.x, w.y, w.z, 1.0f});
+// A triangle clipped by six planes has at most nine corners.
+constexpr uint32_t kPolyMax = 12;
+
+// Clips a polygon held one corner per lane (lanes 0..n-1) by the six planes
+// and returns its number of corners (0 when nothing is left).  Per plane every
+// lane emits its own corner if it is inside and the crossing to the next
+// corner if the edge crosses; the emissions are ordered by two ballots and
+// exchanged through LDS.
+LH_DEV uint32_t clip_polygon(f4& v, uint32_t n, uint32_t lane, float4* poly) {
+    for (int k = 0; k < 6 && n >= 3; k++) {
+        lds_order();
+        if (lane < n) poly[lane] = make_float4(v.x, v.y, v.z, v.w);
+        lds_order();
+        const bool live = lane < n;
+        const float4 q = poly[live && lane + 1 < n ? lane + 1 : 0];
+        const f4 b{q.x, q.y, q.z, q.w};
+        const float da = plane_dist(v, k), db = plane_dist(b, k);
+        const bool ia = da >= 0.0f, ib = db >= 0.0f, keep = live && ia, cross = live && ia != ib;
+        const uint64_t mk = ballot(keep), mc = ballot(cross);
+        const uint32_t at = lanes_below(mk) + lanes_below(mc);
+        lds_order();
+        if (keep) poly[at] = make_float4(v.x, v.y, v.z, v.w);
+        if (cross) {
+            const f4 c = ia ? clip_point(v, b, da, db) : clip_point(b, v, db, da);
+            poly[at + (keep ? 1u : 0u)] = make_float4(c.x, c.y, c.z, c.w);
         }
-        int n = 3;
-        for (int k = 0; k < 6 && n >= 3; k++) {
-            int m = 0;
-            for (int i = 0; i < n; i++) {
-                f4 a = poly[i], b = poly[i + 1 == n ? 0 : i + 1];
-                float da = plane_dist(a, k), db = plane_dist(b, k);
-                bool ia = da >= 0.0f, ib = db >= 0.0f;
-                if (ia) tmp[m++] = a;
-                if (ia != ib) tmp[m++] = ia ? clip_point(a, b, da, db) : clip_point(b, a, db, da);
-            }
-            for (int i = 0; i < m; i++) poly[i] = tmp[i];
-            n = m;
-        }
-        if (n < 3) continue;
-        SV sv[12];
-        bool ok = true;
-        for (int i = 0; i < n; i++) ok = ok && project(poly[i], p.W, p.H, sv[i]);
-        if (!ok) continue;
-        const uint32_t id = (mid << LH_KEY_TRI_BITS) | t;
-        for (int i = 1; i + 1 < n; i++) {
-            SV a = sv[0], b = sv[i], c = sv[i + 1];
-            int64_t area;
-            int32_t xlo, xhi, ylo, yhi, ex, ey;
-            if (!setup<KIND>(a, b, c, p.W, p.H, area, xlo, xhi, ylo, yhi, ex, ey, alpha)) continue;
-            uint32_t slot = atomicAdd(big_counter, 1u);
-            if (slot < v.big_capacity)
-                store_big(qs.big + slot, a, b, c, id, xlo, xhi, ylo, yhi, pi, alpha);
-            else
-                atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
+        lds_order();
+        n = uint32_t(__popcll(mk) + __popcll(mc));
+        if (lane < n) {
+            const float4 c = poly[lane];
+            v = f4{c.x, c.y, c.z, c.w};
         }
     }
+    return n >= 3 ? n : 0u;
 }
 
-// Triangles of the large queue whose pixel box holds at most this many pixels
-// are rasterized by one wave alone; larger ones by the whole block.
+// Triangles over kNarrow whose pixel box holds at most this many pixels are
+// rasterized by one wave alone; larger ones by the whole block.
 constexpr int32_t kWaveBoxPx = 4096;
 
-// Rasterizes the pixels of one queued triangle's box that fall on lanes
-// first, first + stride, ... of the box's row-major pixel order.  Coverage
-// and depth of each pixel are evaluated exactly as in the other paths
-// (64-bit edge functions at the pixel centre, top-left rule).
-template <int KIND, bool ST, bool ALPHA>
-LH_DEV void raster_box(const lh_scene& s, const lh_view& v, const PassSet& ps, const BigTri& b, int32_t first,
-                       int32_t stride, Tally<ST>* tally) {
-    const uint32_t pi = uint32_t(b.xlo) >> 13;
-    const Pass p = make_pass(v, ps.pass0 + pi);
+// float(e), rounded once, for |e| < 2^53: exact as a double first (four
+// instructions; the direct conversion takes a dozen).
+LH_DEV float to_float(int64_t e) {
+    return float(__builtin_fma(double(int32_t(e >> 32)), 4294967296.0, double(uint32_t(e))));
+}
+
+// Rasterizes the pixels of one triangle's box that fall on lanes first,
+// first + stride, ... of the box's row-major pixel order.  Coverage and depth
+// of each pixel are evaluated exactly as in the other paths (64-bit edge
+// functions at the pixel centre, stepped exactly; top-left rule).
+template <int KIND, bool ST, bool ALPHA, class A>
+LH_DEV void raster_box(const lh_scene& s, const lh_view& v, const Pass& p, const BigTri& b, A& alpha, int32_t first,
+                       int32_t stride, Tally<ST>& tally) {
+    if constexpr (ALPHA) {
+        lds_order();
+        if (lane_id() == 0) alpha.store(0, shading::alpha_setup(s, view_matrix<KIND>(v, p.pass), b.id));
+        lds_order();
+    }
     const int32_t X0 = b.X[0], X1 = b.X[1], X2 = b.X[2], Y0 = b.Y[0], Y1 = b.Y[1], Y2 = b.Y[2];
     const int64_t area = edge64(X0, Y0, X1, Y1, X2, Y2);
     const float inv_area = 1.0f / float(area);
     const float z0 = b.z[0], d10 = b.z[1] - b.z[0], d20 = b.z[2] - b.z[0];
-    const bool tl0 = top_left(X1, Y1, X2, Y2), tl1 = top_left(X2, Y2, X0, Y0), tl2 = top_left(X0, Y0, X1, Y1);
+    const int64_t m0 = top_left(X1, Y1, X2, Y2) ? 0 : 1, m1 = top_left(X2, Y2, X0, Y0) ? 0 : 1,
+                  m2 = top_left(X0, Y0, X1, Y1) ? 0 : 1;
     const int32_t xlo = b.xlo & 0x1FFF, xhi = b.xhi, ylo = b.ylo & ~kBigAlpha, yhi = b.yhi;
     const int32_t bw = xhi - xlo + 1, n = bw * (yhi - ylo + 1);
     if (first >= n) return;
-    // Step by `stride` pixels in row-major order: sy rows and sx columns,
-    // plus one row when the column passes the box's right edge.
+    // Step by `stride` pixels in row-major order: sy rows and sx columns, and
+    // one row on and bw columns back when the column passes the right edge.
     const int32_t sy = stride / bw, sx = stride - sy * bw;
     int32_t py = ylo + first / bw, px = xlo + (first - (first / bw) * bw);
+    const int32_t Px = px * 256 + 128, Py = py * 256 + 128;
+    int64_t e0 = edge64(X1, Y1, X2, Y2, Px, Py), e1 = edge64(X2, Y2, X0, Y0, Px, Py), e2 = edge64(X0, Y0, X1, Y1, Px, Py);
+    const int64_t c0 = -256ll * (Y2 - Y1), r0 = 256ll * (X2 - X1), c1 = -256ll * (Y0 - Y2), r1 = 256ll * (X0 - X2),
+                  c2 = -256ll * (Y1 - Y0), r2 = 256ll * (X1 - X0);
+    const int64_t a0 = sx * c0 + sy * r0, a1 = sx * c1 + sy * r1, a2 = sx * c2 + sy * r2;
+    const int64_t w0 = r0 - bw * c0, w1 = r1 - bw * c1, w2 = r2 - bw * c2;
     for (int32_t i = first; i < n; i += stride) {
-        const int32_t Px = px * 256 + 128, Py = py * 256 + 128;
-        const int64_t e0 = edge64(X1, Y1, X2, Y2, Px, Py);
-        const int64_t e1 = edge64(X2, Y2, X0, Y0, Px, Py);
-        const int64_t e2 = edge64(X0, Y0, X1, Y1, Px, Py);
-        const bool in = (e0 > 0 || (e0 == 0 && tl0)) && (e1 > 0 || (e1 == 0 && tl1)) && (e2 > 0 || (e2 == 0 && tl2));
-        if (in && (!ALPHA || alpha_pass<KIND>(s, v, p, b.id, px, py))) {
-            const float l1 = float(e1) * inv_area, l2 = float(e2) * inv_area;
-            const bool issued = fragment<KIND>(p, px, py, (z0 + l1 * d10) + l2 * d20, b.id);
-#pragma unroll
-            for (uint32_t q = 0; q < LH_NUM_CASCADES; q++)
-                if (q == pi) tally[q].hit(issued);
+        if (e0 >= m0 && e1 >= m1 && e2 >= m2) {
+            const float l1 = to_float(e1) * inv_area, l2 = to_float(e2) * inv_area;
+            fragment<KIND, ST, !ST>(p, px, py, (z0 + l1 * d10) + l2 * d20, b.id, tally, [&] {
+                if constexpr (ALPHA)
+                    return shading::alpha_at(s, alpha.load(0), p.W, p.H, px, py);
+                else
+                    return true;
+            });
         }
-        px += sx;
-        py += sy;
+        px += sx, py += sy;
+        e0 += a0, e1 += a1, e2 += a2;
         if (px > xhi) {
-            px -= bw;
-            py++;
+            px -= bw, py++;
+            e0 += w0, e1 += w1, e2 += w2;
         }
     }
 }
 
-// View blockIdx.z.  Each round the block takes four queue entries, one per
-// wave.  A wave rasterizes its own triangle when the box is at most
-// kWaveBoxPx pixels (most of the queue: slivers just over the medium extent),
-// so a 54-pixel box costs one wave pass instead of a 256-thread block; the
-// larger boxes of the round are rasterized by all four waves together first.
-// ALPHA selects the entries of alpha-clip geometry (alpha test per sample),
-// so the opaque instantiation keeps its small register footprint; the alpha
-// one returns at once when the view's culls counted no alpha-clip draw.
+// The clip-crossing and the large triangles of view blockIdx.z.
+//
+// Large triangles: a wave takes up to 64 queue entries at a time.  Those within kNarrow (most of the
+// queue: triangles just over the medium extent) go through raster_queue
+// together, pass by pass; a wider one is rasterized by its wave alone when its
+// box holds at most kWaveBoxPx pixels, and by the block's four waves together
+// above.  Clip-crossing triangles: a block takes one at a time; its waves all
+// clip it (they need no exchange to agree) and share the pieces of the fan:
+// a narrow piece goes to one wave, a wide one to the whole block.
+//
+// ALPHA selects the entries of alpha-clip geometry (alpha test per sample), so
+// the opaque instantiation keeps its small register footprint; the alpha one
+// returns at once when the view's culls counted no alpha-clip draw.
+//
+// Bound by the depth atomics (20 M samples of the 4K field in 306 k wave
+// instructions) until the target is read first, which leaves a third of them.
+// 3840x2160, 220 k queued triangles: 215 us when every triangle walked its box
+// alone with 64-bit edges, 556 with four-pixel runs per lane (a wave's atomics
+// on 64 rows at once) and contiguous entries, 401 with single pixels, 181 with
+// the entries dealt out, 120 with the early test, 111 on 4,096 blocks.
 template <int KIND, class VS, bool ST, bool ALPHA>
-__global__ void __launch_bounds__(256) k_raster_big(lh_scene s, VS vs, PassSet ps) {
+__global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big(lh_scene s, VS vs, PassSet ps) {
     const lh_view& v = vs.get(blockIdx.z);
     if constexpr (ALPHA) {
         uint32_t n = 0;
         for (uint32_t k = 0; k < ps.n; k++) n += v.counters[LH_CNT_ALPHA_DRAWS + ps.pass0 + k];
         if (n == 0) return;
     }
-    const Queues qs = queues(v);
     const uint32_t count = min(v.counters[LH_CNT_BIG + ps.pass0], v.big_capacity);
-    const uint32_t wave = threadIdx.x >> 6;
-    // wide[r & 1][w]: wave w's triangle of round r goes to the whole block.
-    // Two buffers, because a wave may write round r + 1's flag while another
-    // still reads round r's (no wave gets two rounds ahead: each round has a
-    // barrier).
-    __shared__ uint32_t wide[2][4];
-    // Statistics: each lane counts per pass of the set over all of the
-    // block's triangles, and the wave adds them to the view's counters once
-    // at the end (a flush per triangle also measured wrong depths on the
-    // large frame's sliver triangles with statistics on).
-    Tally<ST> tally[LH_NUM_CASCADES];
+    const uint32_t clips = min(v.counters[LH_CNT_CLIP + ps.pass0], v.clip_capacity);
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    __shared__ TriQueueOf<64> queues4[4];
+    __shared__ float4 poly4[4][kPolyMax];
+    // giant[r & 1][w]: wave w's entries of round r for the whole block.  Two
+    // buffers, because a wave may write round r + 1's mask while another still
+    // reads round r's (no wave gets two rounds ahead: each has a barrier).
+    __shared__ uint64_t giant[2][4];
+    TriQueueOf<64>& queue = queues4[wave];
+    __shared__ std::conditional_t<ALPHA, AlphaStore, NoAlpha> alphas4[4];
+    auto& alpha = alphas4[wave];
+    const Queues qs = queues(v);
+    Tally<ST> tally;
+    auto raster_narrow = [&](uint32_t n, const Pass& p) {
+        LhMat4 M{};
+        if constexpr (ALPHA) M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
+        raster_queue<KIND, ST, ALPHA, !ST>(s, M, p, queue, alpha, 0, n, lane, tally);
+        lds_order();
+        tally.flush(v, p.pass);
+    };
+    // Entry of lane l of wave w in the round that starts at b0.  Neighbours in
+    // the queue are neighbours on a mesh and of much the same size, so a
+    // wave's entries lie `waves` apart: a run of large ones is shared out.
+    const uint32_t waves = gridDim.x * 4;
+    auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + blockIdx.x * 4 + w + l * waves; };
     uint32_t round = 0;
-    for (uint32_t e0 = blockIdx.x * 4; e0 < count; e0 += gridDim.x * 4, round ^= 1) {  // block-uniform
-        const uint32_t e = e0 + wave;
-        bool own = false, shared = false;
-        BigTri b;
-        if (e < count) {
-            b = qs.big[e];
-            if (((b.ylo & kBigAlpha) != 0) == ALPHA) {
-                const int32_t bw = b.xhi - (b.xlo & 0x1FFF) + 1, bh = b.yhi - (b.ylo & ~kBigAlpha) + 1;
-                own = bw * bh <= kWaveBoxPx;
-                shared = !own;
-            }
+    for (uint32_t b0 = 0; b0 + blockIdx.x * 4 < count; b0 += 64 * waves, round ^= 1) {  // block-uniform
+        const uint32_t e = entry(b0, wave, lane);
+        BigTri b{};
+        const bool mine = e < count;
+        if (mine) b = qs.big[e];
+        const int32_t xlo = b.xlo & 0x1FFF, ylo = b.ylo & ~kBigAlpha;
+        const uint32_t pi = uint32_t(b.xlo) >> 13;
+        const int32_t extent = max(max(b.X[0], max(b.X[1], b.X[2])) - min(b.X[0], min(b.X[1], b.X[2])),
+                                   max(b.Y[0], max(b.Y[1], b.Y[2])) - min(b.Y[0], min(b.Y[1], b.Y[2])));
+        const bool drawn = mine && ((b.ylo & kBigAlpha) != 0) == ALPHA;
+        const bool wide = drawn && extent > kNarrow;
+        const bool huge = wide && (b.xhi - xlo + 1) * (b.yhi - ylo + 1) > kWaveBoxPx;
+        for (uint32_t q = 0; q < ps.n; q++) {
+            const bool now = drawn && !wide && pi == q;
+            const uint64_t m = ballot(now);
+            if (m == 0) continue;
+            if (now)
+                queue.store(lanes_below(m), xlo, ylo, SV{b.X[0], b.Y[0], b.z[0]}, SV{b.X[1], b.Y[1], b.z[1]},
+                            SV{b.X[2], b.Y[2], b.z[2]}, b.id);
+            raster_narrow(uint32_t(__popcll(m)), make_pass(v, ps.pass0 + q));
         }
-        if (lane_id() == 0) wide[round][wave] = shared ? 1u : 0u;
+        for (uint64_t m = ballot(wide && !huge); m; m &= m - 1) {
+            const BigTri t = qs.big[entry(b0, wave, first_lane(m))];
+            const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
+            raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, int32_t(lane), 64, tally);
+            tally.flush(v, p.pass);
+        }
+        const uint64_t hm = ballot(huge);
+        if (lane == 0) giant[round][wave] = hm;
         __syncthreads();
         for (uint32_t w = 0; w < 4; w++)
-            if (wide[round][w]) raster_box<KIND, ST, ALPHA>(s, v, ps, qs.big[e0 + w], threadIdx.x, 256, tally);
-        if (own) raster_box<KIND, ST, ALPHA>(s, v, ps, b, int32_t(lane_id()), 64, tally);
+            for (uint64_t m = giant[round][w]; m; m &= m - 1) {
+                const BigTri t = qs.big[entry(b0, w, first_lane(m))];
+                const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
+                raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, int32_t(threadIdx.x), 256, tally);
+                tally.flush(v, p.pass);
+            }
     }
-#pragma unroll
-    for (uint32_t q = 0; q < LH_NUM_CASCADES; q++)
-        if (q < ps.n) tally[q].flush(v, ps.pass0 + q);
+    for (uint32_t c = blockIdx.x; c < clips; c += gridDim.x) {
+        const uint2 e = qs.clip[c];
+        if (((e.y & kClipAlpha) != 0) != ALPHA) continue;
+        const uint32_t d = e.x >> LH_KEY_TRI_BITS, t = e.x & ((1u << LH_KEY_TRI_BITS) - 1), pi = e.y & ~kClipAlpha;
+        const Pass p = make_pass(v, ps.pass0 + pi);
+        const MeshletReference ref = p.draws[d];
+        const Instance& in = s.instances[ref.instance_index];
+        const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
+        const Meshlet& ml = ptr<Meshlet>(mi.meshlets)[ref.meshlet_index];
+        const uint32_t mid = s.instance_meshlet_base[ref.instance_index] + ref.meshlet_index;
+        f4 corner{0, 0, 0, 0};
+        if (lane < 3) {
+            const uint32_t micro = ptr<uint8_t>(mi.micro_indices)[ml.triangle_offset + 3 * t + lane];
+            const f3 w = mat4_point(in.transform, load_position(mi, load_index(mi, ml.index_offset + micro)));
+            corner = mat4_mul_vec4(view_matrix<KIND>(v, p.pass), f4{w.x, w.y, w.z, 1.0f});
+        }
+        const uint32_t n = clip_polygon(corner, 3, lane, poly4[wave]);
+        SV sv{0, 0, 0.0f};
+        const bool ok = lane >= n || project(corner, p.W, p.H, sv);
+        if (n == 0 || ballot(!ok) != 0) continue;
+        // piece i of the fan (lanes 1..n-2): corners 0, i, i + 1
+        const uint32_t after = min(lane + 1, 63u);
+        SV v0{__shfl(sv.X, 0, 64), __shfl(sv.Y, 0, 64), __shfl(sv.z, 0, 64)}, v1 = sv,
+           v2{__shfl(sv.X, int(after), 64), __shfl(sv.Y, int(after), 64), __shfl(sv.z, int(after), 64)};
+        int64_t area;
+        int32_t xlo, xhi, ylo, yhi, ex, ey;
+        const bool set = setup<KIND>(v0, v1, v2, p.W, p.H, area, xlo, xhi, ylo, yhi, ex, ey, ALPHA);
+        const bool piece = set && lane >= 1 && lane + 1 < n;
+        const bool wide = piece && max(ex, ey) > kNarrow;
+        const uint32_t id = (mid << LH_KEY_TRI_BITS) | t;
+        const bool narrow = piece && !wide && (lane & 3u) == wave;
+        const uint64_t nm = ballot(narrow);
+        if (nm) {
+            if (narrow) queue.store(lanes_below(nm), xlo, ylo, v0, v1, v2, id);
+            raster_narrow(uint32_t(__popcll(nm)), p);
+        }
+        for (uint64_t m = ballot(wide); m; m &= m - 1) {
+            const uint32_t l = first_lane(m);
+            BigTri b;
+            b.X[0] = readlane(v0.X, l), b.X[1] = readlane(v1.X, l), b.X[2] = readlane(v2.X, l);
+            b.Y[0] = readlane(v0.Y, l), b.Y[1] = readlane(v1.Y, l), b.Y[2] = readlane(v2.Y, l);
+            b.z[0] = readlane(v0.z, l), b.z[1] = readlane(v1.z, l), b.z[2] = readlane(v2.z, l);
+            b.id = id;
+            b.xlo = uint16_t(readlane(xlo, l)), b.ylo = uint16_t(readlane(ylo, l));
+            b.xhi = uint16_t(readlane(xhi, l)), b.yhi = uint16_t(readlane(yhi, l));
+            raster_box<KIND, ST, ALPHA>(s, v, p, b, alpha, int32_t(threadIdx.x), 256, tally);
+            tally.flush(v, p.pass);
+        }
+    }
 }
 
 // Batch plan: off[k + 1] = off[k] + surviving meshlets of segment k
@@ -394,8 +481,8 @@ namespace lhk {
 // (tile.hip) when its tuning class asks for it; the per-meshlet kernel then
 // covers only the draws it left.
 template <int KIND, bool ST, class VS>
-hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const RasterTuning& t, uint32_t clip_blocks,
-                          uint32_t big_blocks, hipStream_t st) {
+hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const RasterTuning& t, uint32_t big_blocks,
+                          hipStream_t st) {
     const uint32_t nv = vs.count();
     bool tiled = false;
     if constexpr (std::is_same<VS, OneView>::value)
@@ -410,16 +497,21 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
     } else {
         mark(KIND == 0 ? "raster_meshlets_view" : "raster_meshlets_shadow", st);
     }
-    hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs, ps);
+    // The draw count is on the device; the scene's meshlets bound what a pass
+    // can draw (a block without a draw still costs its launch: 24,576 empty
+    // ones 4 us).  The direct list is short or empty.
+    const uint64_t most = uint64_t(std::max(s.total_meshlets, 1u)) * nv;
+    const uint32_t blocks = uint32_t(std::min<uint64_t>(t.meshlet_blocks, most));
+    hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST>), dim3(tiled ? std::min(blocks, 1024u) : blocks), dim3(64), 0,
+                       st, s, vs, ps);
     ps.direct = 0;
     const bool alpha = !(s.flags & LH_SCENE_OPAQUE_ONLY);
     if (alpha) {
         mark(KIND == 0 ? "raster_alpha_view" : "raster_alpha_shadow", st);
-        hipLaunchKernelGGL((k_raster_alpha<KIND, VS, ST>), dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs,
-                           ps);
+        PassSet pa = ps;
+        pa.medium_extent = std::min(ps.medium_extent, kAlphaMediumPx * 256);
+        hipLaunchKernelGGL((k_raster_alpha<KIND, VS, ST>), dim3(blocks), dim3(64), 0, st, s, vs, pa);
     }
-    mark(KIND == 0 ? "raster_clip_view" : "raster_clip_shadow", st);
-    hipLaunchKernelGGL((k_raster_clip<KIND, VS>), dim3(clip_blocks, 1, nv), dim3(64), 0, st, s, vs, ps);
     mark(KIND == 0 ? "raster_big_view" : "raster_big_shadow", st);
     hipLaunchKernelGGL((k_raster_big<KIND, VS, ST, false>), dim3(big_blocks, 1, nv), dim3(256), 0, st, s, vs, ps);
     if (alpha) {
@@ -431,15 +523,15 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
 
 // Statistics are a single-view feature (LH_VIEW_STATISTICS).
 template <int KIND>
-hipError_t launch_set(const lh_scene& s, const OneView& vs, const PassSet& ps, const RasterTuning& t, uint32_t cb,
-                      uint32_t bb, hipStream_t st) {
-    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, cb, bb, st);
-    return launch_kernels<KIND, false>(s, vs, ps, t, cb, bb, st);
+hipError_t launch_set(const lh_scene& s, const OneView& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
+                      hipStream_t st) {
+    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, bb, st);
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, st);
 }
 template <int KIND>
-hipError_t launch_set(const lh_scene& s, const ViewTable& vs, const PassSet& ps, const RasterTuning& t, uint32_t cb,
-                      uint32_t bb, hipStream_t st) {
-    return launch_kernels<KIND, false>(s, vs, ps, t, cb, bb, st);
+hipError_t launch_set(const lh_scene& s, const ViewTable& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
+                      hipStream_t st) {
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, st);
 }
 
 template <class VS>
@@ -456,11 +548,10 @@ hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npas
     const uint32_t medium_px = std::min<uint32_t>(std::max(medium_sel, small_px), 64);
     PassSet ps{pass0, npasses, int32_t(small_px * 256), int32_t(medium_px * 256), phase2 ? 1u : 0u, 0u};
     const uint32_t nv = vs.count();
-    // per-view persistent grids of the queue kernels shrink with the batch size
-    const uint32_t clip_blocks = nv > 1 ? std::max(t.clip_blocks / 16, 4u) : t.clip_blocks;
+    // the per-view persistent grid of the queue kernel shrinks with the batch size
     const uint32_t big_blocks = nv > 1 ? std::max(t.big_blocks / 16, 32u) : t.big_blocks;
-    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, clip_blocks, big_blocks, st);
-    return launch_set<1>(s, vs, ps, t, clip_blocks, big_blocks, st);
+    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, big_blocks, st);
+    return launch_set<1>(s, vs, ps, t, big_blocks, st);
 }
 
 template hipError_t raster<OneView>(const lh_scene&, const OneView&, uint32_t, uint32_t, const RasterTuning&,

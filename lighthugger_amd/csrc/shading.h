@@ -50,18 +50,33 @@ struct BaryDeriv {
     f3 lambda, ddx, ddy;
 };
 
-// CalcFullBary (src/shaders/common/vbuffer.glsl:11-63).
-LH_DEV BaryDeriv calc_full_bary(f4 p0, f4 p1, f4 p2, f2 ndc, f2 win) {
-    BaryDeriv r;
-    const f3 invW{1.0f / p0.w, 1.0f / p1.w, 1.0f / p2.w};
-    const f2 n0{p0.x * invW.x, p0.y * invW.x}, n1{p1.x * invW.y, p1.y * invW.y}, n2{p2.x * invW.z, p2.y * invW.z};
+// CalcFullBary (src/shaders/common/vbuffer.glsl:11-63), in two parts: what
+// depends on the triangle alone, and the barycentrics and their derivatives at
+// one point.
+struct BarySetup {
+    f3 invW;
+    f2 n0;
+    f3 ddx, ddy;  // per unit of ndc
+};
+LH_DEV BarySetup bary_setup(f4 p0, f4 p1, f4 p2) {
+    BarySetup b;
+    b.invW = f3{1.0f / p0.w, 1.0f / p1.w, 1.0f / p2.w};
+    b.n0 = f2{p0.x * b.invW.x, p0.y * b.invW.x};
+    const f2 n0 = b.n0, n1{p1.x * b.invW.y, p1.y * b.invW.y}, n2{p2.x * b.invW.z, p2.y * b.invW.z};
     const f2 c0{n2.x - n1.x, n2.y - n1.y}, c1{n0.x - n1.x, n0.y - n1.y};
     const float invDet = 1.0f / (c0.x * c1.y - c1.x * c0.y);
-    r.ddx = mul(mul(f3{n1.y - n2.y, n2.y - n0.y, n0.y - n1.y}, invDet), invW);
-    r.ddy = mul(mul(f3{n2.x - n1.x, n0.x - n2.x, n1.x - n0.x}, invDet), invW);
+    b.ddx = mul(mul(f3{n1.y - n2.y, n2.y - n0.y, n0.y - n1.y}, invDet), b.invW);
+    b.ddy = mul(mul(f3{n2.x - n1.x, n0.x - n2.x, n1.x - n0.x}, invDet), b.invW);
+    return b;
+}
+LH_DEV BaryDeriv bary_at(const BarySetup& b, f2 ndc, f2 win) {
+    BaryDeriv r;
+    const f3 invW = b.invW;
+    r.ddx = b.ddx;
+    r.ddy = b.ddy;
     float ddxSum = (r.ddx.x + r.ddx.y) + r.ddx.z;
     float ddySum = (r.ddy.x + r.ddy.y) + r.ddy.z;
-    const f2 dv{ndc.x - n0.x, ndc.y - n0.y};
+    const f2 dv{ndc.x - b.n0.x, ndc.y - b.n0.y};
     const float interpInvW = (invW.x + dv.x * ddxSum) + dv.y * ddySum;
     const float interpW = 1.0f / interpInvW;
     r.lambda.x = interpW * ((invW.x + dv.x * r.ddx.x) + dv.y * r.ddy.x);
@@ -83,6 +98,7 @@ LH_DEV BaryDeriv calc_full_bary(f4 p0, f4 p1, f4 p2, f2 ndc, f2 win) {
                wdy * (r.lambda.z * interpInvW + r.ddy.z) - r.lambda.z};
     return r;
 }
+LH_DEV BaryDeriv calc_full_bary(f4 p0, f4 p1, f4 p2, f2 ndc, f2 win) { return bary_at(bary_setup(p0, p1, p2), ndc, win); }
 
 LH_DEV f3 interp1(const BaryDeriv& d, float a, float b, float c) {
     const f3 m{a, b, c};
@@ -475,38 +491,52 @@ LH_DEV bool decode(const lh_scene& s, const lh_view& v, uint64_t key, Surface& s
 // :130-145): the base-colour texture's alpha at the pixel centre, discarded
 // below 0.5.  The uv is interpolated perspective-correctly and its LOD taken
 // from the analytic derivatives (CalcFullBary, as the resolve does) in place
-// of the hardware's 2x2-quad differences.  `m` is the pass's view-projection
-// matrix, W x H its target; the triangle is the one the key id names.  A
-// triangle with a vertex at or behind w = 0, or a non-finite uv, passes.
-LH_DEV bool alpha_visible(const lh_scene& s, const LhMat4& m, uint32_t W, uint32_t H, uint32_t id, int32_t px,
-                          int32_t py) {
+// of the hardware's 2x2-quad differences.  A triangle with a vertex at or
+// behind w = 0, or a non-finite uv, passes.
+//
+// What the test needs of a triangle, fetched and transformed once for all its
+// samples; `texture` is UNUSED_TEXTURE_INDEX when every sample passes.
+struct AlphaTri {
+    BarySetup bary;
+    f2 uv[3], offset;
+    uint32_t texture;
+};
+// `m` is the pass's view-projection matrix; the triangle is the one the key id
+// names.
+LH_DEV AlphaTri alpha_setup(const lh_scene& s, const LhMat4& m, uint32_t id) {
+    AlphaTri t;
     const MeshletReference ref = s.meshlet_table[id >> LH_KEY_TRI_BITS];
     const Instance& in = s.instances[ref.instance_index];
     const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
-    if (!has_texture(s, mi.base_color_texture_index)) return true;  // white, alpha 1
     const Meshlet& ml = ptr<Meshlet>(mi.meshlets)[ref.meshlet_index];
     const uint8_t* micro = ptr<uint8_t>(mi.micro_indices) + ml.triangle_offset + 3 * (id & ((1u << LH_KEY_TRI_BITS) - 1));
     const f2 ts{mi.texture_scale.x, mi.texture_scale.y};
+    t.offset = {mi.texture_offset.x, mi.texture_offset.y};
+    // an index without a texture reads as white, alpha 1
+    t.texture = has_texture(s, mi.base_color_texture_index) ? mi.base_color_texture_index : UNUSED_TEXTURE_INDEX;
     f4 clip[3];
-    f2 uvs[3];
     for (int j = 0; j < 3; j++) {
         const uint32_t vi = load_index(mi, ml.index_offset + micro[j]);
         const f3 w = mat4_point(in.transform, load_position(mi, vi));
         clip[j] = mat4_mul_vec4(m, f4{w.x, w.y, w.z, 1.0f});
-        if (!(clip[j].w > 0.0f)) return true;
-        const f2 t = load_uv(mi, vi);
-        uvs[j] = {t.x * ts.x, t.y * ts.y};
+        if (!(clip[j].w > 0.0f)) t.texture = UNUSED_TEXTURE_INDEX;
+        const f2 q = load_uv(mi, vi);
+        t.uv[j] = {q.x * ts.x, q.y * ts.y};
     }
+    t.bary = bary_setup(clip[0], clip[1], clip[2]);
+    return t;
+}
+LH_DEV bool alpha_at(const lh_scene& s, const AlphaTri& t, uint32_t W, uint32_t H, int32_t px, int32_t py) {
+    if (t.texture == UNUSED_TEXTURE_INDEX) return true;
     const f2 win{float(W), float(H)};
     const f2 ndc{(float(px) + 0.5f) / win.x * 2.0f - 1.0f, (float(py) + 0.5f) / win.y * 2.0f - 1.0f};
-    const BaryDeriv bary = calc_full_bary(clip[0], clip[1], clip[2], ndc, win);
-    Interp2 uv = interp2(bary, uvs[0], uvs[1], uvs[2]);
-    uv.v.x += mi.texture_offset.x;
-    uv.v.y += mi.texture_offset.y;
+    Interp2 uv = interp2(bary_at(t.bary, ndc, win), t.uv[0], t.uv[1], t.uv[2]);
+    uv.v.x += t.offset.x;
+    uv.v.y += t.offset.y;
     if (!(isfinite(uv.v.x) && isfinite(uv.v.y) && isfinite(uv.dx.x) && isfinite(uv.dx.y) && isfinite(uv.dy.x) &&
           isfinite(uv.dy.y)))
         return true;
-    return !(sample_texture(s, mi.base_color_texture_index, uv).w < 0.5f);
+    return !(sample_texture(s, t.texture, uv).w < 0.5f);
 }
 
 // Differentiable parameters: each pointer, when set, replaces the value the

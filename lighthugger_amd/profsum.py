@@ -31,13 +31,11 @@ FRAME_KERNELS = {
     "bin_fill_view": "k_bin_fill",
     # with the tiled raster on, the per-meshlet kernel of the main view runs as
     # raster_direct_view (the draws the bins left); otherwise as raster_meshlets_view
-    "raster_direct_view": "k_raster_meshlets<0, lhd::OneView, false, false>",
-    "raster_meshlets_view": "k_raster_meshlets<0, lhd::OneView, false, false>",
-    "raster_meshlets_shadow": "k_raster_meshlets<1, lhd::OneView, false, false>",
+    "raster_direct_view": "k_raster_meshlets<0, lhd::OneView, false>",
+    "raster_meshlets_view": "k_raster_meshlets<0, lhd::OneView, false>",
+    "raster_meshlets_shadow": "k_raster_meshlets<1, lhd::OneView, false>",
     "raster_big_view": "k_raster_big<0, lhd::OneView, false, false>",
     "raster_big_shadow": "k_raster_big<1, lhd::OneView, false, false>",
-    "raster_clip_view": "k_raster_clip<0, lhd::OneView>",
-    "raster_clip_shadow": "k_raster_clip<1, lhd::OneView>",
     "resolve": "k_resolve",
     "depth_bounds": "k_depth_bounds<lhd::OneView>",
     "fit_cull_instances_shadow": "k_fit_cull_instances_shadow<lhd::OneView>",
