@@ -329,12 +329,42 @@ LH_DEV uint32_t wrap_index(int32_t i, int32_t n) {
 struct TexelQuad {
     f4 t00, t10, t01, t11;
 };
+// The two texels (x, j), (x + 1 mod w, j) of a plain RGBA8 level: neighbours in
+// memory, so one 8-byte load; the row's last texel takes its wrapped neighbour
+// by itself.
+LH_DEV uint2 texel_pair(const uint32_t* row, uint32_t w, uint32_t x) {
+    if (w == 1) return make_uint2(row[0], row[0]);
+    const uint32_t from = min(x, w - 2);
+    uint2 p;
+    __builtin_memcpy(&p, row + from, 8);
+    if (x != from) p = make_uint2(p.y, row[0]);
+    return p;
+}
 LH_DEV TexelQuad texel_quad(const LhTexture& t, uint32_t level, int32_t w, int32_t h, int32_t i, int32_t j) {
     const uint32_t i0 = wrap_index(i, w), j0 = wrap_index(j, h);
     const uint32_t i1 = i0 + 1 == uint32_t(w) ? 0u : i0 + 1, j1 = j0 + 1 == uint32_t(h) ? 0u : j0 + 1;
     const uint32_t W = uint32_t(w);
-    return {unpack_texel(t, texel_rgba8(t, level, W, i0, j0)), unpack_texel(t, texel_rgba8(t, level, W, i1, j0)),
-            unpack_texel(t, texel_rgba8(t, level, W, i0, j1)), unpack_texel(t, texel_rgba8(t, level, W, i1, j1))};
+    if ((t.format & (LH_TEXTURE_FORMAT_MASK | LH_TEXTURE_SRGB)) == LH_TEXTURE_RGBA8) {
+        const uint32_t* base = ptr<uint32_t>(t.texels) + t.level_offset[level];
+        const uint2 p0 = texel_pair(base + size_t(j0) * W, W, i0), p1 = texel_pair(base + size_t(j1) * W, W, i0);
+        auto texel = [](uint32_t p) {
+            return f4{unorm8(p & 255u), unorm8((p >> 8) & 255u), unorm8((p >> 16) & 255u), unorm8(p >> 24)};
+        };
+        return {texel(p0.x), texel(p0.y), texel(p1.x), texel(p1.y)};
+    }
+    // Block and sRGB formats: one copy of the decoders, run for one texel after
+    // the other (unrolled for every texel, level and texture they were nine
+    // tenths of the resolve's code).
+    TexelQuad q;
+#pragma unroll 1
+    for (int k = 0; k < 4; k++) {
+        const f4 v = unpack_texel(t, texel_rgba8(t, level, W, (k & 1) ? i1 : i0, (k & 2) ? j1 : j0));
+        if (k == 0) q.t00 = v;
+        if (k == 1) q.t10 = v;
+        if (k == 2) q.t01 = v;
+        if (k == 3) q.t11 = v;
+    }
+    return q;
 }
 LH_DEV f4 bilinear(const LhTexture& t, uint32_t level, f2 uv) {
     const int32_t wi = int32_t(max(1u, t.width >> level)), hi = int32_t(max(1u, t.height >> level));
@@ -576,39 +606,45 @@ LH_DEV float shadow_factor(const lh_view& v, const MeshInfo& mi, f3 world, uint3
     const float S = float(v.shadow_size);
     const float ref = sc.z - bias;
     // The nine taps' 2x2 cells normally tile the 4x4 texels around the centre
-    // tap's cell: those 16 comparisons are made once (a bit each), and a tap
-    // uses them when its own cell, computed exactly as shadow_tap computes
-    // it, is the expected one; a tap that rounding puts elsewhere reads its
-    // own texels.  The sum is the same, bit for bit.
+    // tap's cell: their comparisons are made once, and the taps share them and
+    // the blends along the rows (an x-blend per column offset and row, a
+    // y-blend per tap; with comparisons of 0 or 1 a blend's products are
+    // selections).  Where rounding puts any tap's cell elsewhere, or the
+    // footprint leaves the map, the taps are evaluated one by one.  The sum is
+    // the same, bit for bit.
     const int32_t N = int32_t(v.shadow_size);
     const uint32_t* map = v.shadow_maps + size_t(layer) * v.shadow_size * v.shadow_size;
     const int32_t i0 = int32_t(floorf(sc.x * S - 0.5f)), j0 = int32_t(floorf(sc.y * S - 0.5f));
-    uint32_t lit = 0;  // bit 4 dy + dx: texel (i0 - 1 + dx, j0 - 1 + dy) passes the compare
+    float a[3], b[3];
+    bool tiled = i0 >= 1 && j0 >= 1 && i0 <= N - 3 && j0 <= N - 3;
 #pragma unroll
-    for (int dy = 0; dy < 4; dy++) {
-        const int32_t y = min(max(j0 - 1 + dy, 0), N - 1);
-#pragma unroll
-        for (int dx = 0; dx < 4; dx++) {
-            const int32_t x = min(max(i0 - 1 + dx, 0), N - 1);
-            lit |= (ref < __uint_as_float(map[size_t(y) * uint32_t(N) + uint32_t(x)]) ? 1u : 0u) << (4 * dy + dx);
-        }
+    for (int o = -1; o <= 1; o++) {
+        const float u = (sc.x + float(o) / S) * S - 0.5f, w = (sc.y + float(o) / S) * S - 0.5f;
+        const float fu = floorf(u), fw = floorf(w);
+        tiled = tiled && int32_t(fu) == i0 + o && int32_t(fw) == j0 + o;
+        a[o + 1] = u - fu;
+        b[o + 1] = w - fw;
     }
+    if (tiled) {
+        float blend[3][4];  // [column offset][row]
 #pragma unroll
-    for (int ox = -1; ox <= 1; ox++)
+        for (int r = 0; r < 4; r++) {
+            float4 q;
+            __builtin_memcpy(&q, map + uint32_t(j0 - 1 + r) * uint32_t(N) + uint32_t(i0 - 1), 16);
+            const bool lit[4] = {ref < q.x, ref < q.y, ref < q.z, ref < q.w};
 #pragma unroll
-        for (int oy = -1; oy <= 1; oy++) {
-            const f2 uv{sc.x + float(ox) / S, sc.y + float(oy) / S};
-            const float u = uv.x * S - 0.5f, w = uv.y * S - 0.5f;
-            const float fu = floorf(u), fw = floorf(w);
-            if (int32_t(fu) == i0 + ox && int32_t(fw) == j0 + oy) {
-                const float a = u - fu, b = w - fw;
-                const int k = 4 * (oy + 1) + (ox + 1);
-                auto bit = [&](int q) { return float((lit >> q) & 1u); };
-                shadow_sum += mixf(mixf(bit(k), bit(k + 1), a), mixf(bit(k + 4), bit(k + 5), a), b);
-            } else {
-                shadow_sum += shadow_tap(v, layer, uv, ref);
-            }
+            for (int o = 0; o < 3; o++)
+                blend[o][r] = (lit[o] ? 1.0f - a[o] : 0.0f) + (lit[o + 1] ? a[o] : 0.0f);
         }
+#pragma unroll
+        for (int ox = 0; ox < 3; ox++)
+#pragma unroll
+            for (int oy = 0; oy < 3; oy++) shadow_sum += mixf(blend[ox][oy], blend[ox][oy + 1], b[oy]);
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < 9; k++)
+            shadow_sum += shadow_tap(v, layer, f2{sc.x + float(k / 3 - 1) / S, sc.y + float(k % 3 - 1) / S}, ref);
+    }
     shadow_sum /= 9.0f;
     if (sc.z > 1.0f) shadow_sum = 1.0f;
     return shadow_sum;
@@ -720,8 +756,8 @@ LH_DEV f3 temperature(float t) {
 constexpr float kClockHeatScale = 65000.0f;
 
 LH_DEV f3 resolve_pixel(const lh_scene& s, const lh_view& v, uint32_t x, uint32_t y, const lh_resolve_params& prm) {
-    const uint64_t start_time = clock64();
     const Uniforms& u = *v.uniforms;
+    const uint64_t start_time = u.debug == UNIFORMS_DEBUG_SHADER_CLOCK ? clock64() : 0;
     const f2 win{float(u.window_size.x), float(u.window_size.y)};
     const f2 ndc{float(x) / win.x * 2.0f - 1.0f, float(y) / win.y * 2.0f - 1.0f};  // pixel corner
     Surface sf;
@@ -748,16 +784,8 @@ LH_DEV f3 resolve_pixel(const lh_scene& s, const lh_view& v, uint32_t x, uint32_
     const f3 gn = cross3(sub(sf.pos[1], sf.pos[0]), sub(sf.pos[2], sf.pos[0]));
     const bool flip = dot3(gn, view_vector) < 0.0f;
     if (flip) nrm = neg(nrm);
-    uint32_t cascade = 0;
-    const float shadow_sum = shadow_factor(v, mi, world.v, &cascade);
-    const Lod lod_b = lod_of(s, mi.base_color_texture_index, uv), lod_m = lod_of(s, mi.metallic_roughness_texture_index, uv);
-    if (prm.frozen)
-        reinterpret_cast<uint4*>(prm.frozen)[size_t(y) * v.width + x] = pack_frozen(shadow_sum, flip, lod_b, lod_m);
-    const f4 bc = sample_texture_lod(s, mi.base_color_texture_index, lod_b, uv);
-    const f3 base = mul(f3{bc.x, bc.y, bc.z}, param_base_color(prm, mi, sf.mesh_info));
-    const f4 mr = sample_texture_lod(s, mi.metallic_roughness_texture_index, lod_m, uv);
-    const float roughness = mr.y * param_roughness(prm, s, sf.mesh_info);
-    const float metallic = mr.z * param_metallic(prm, s, sf.mesh_info);
+    // (before the shadow and the other textures: it is the last use of the
+    // position's derivatives)
     if (mi.normal_texture_index != UNUSED_TEXTURE_INDEX) {
         const f4 mn = sample_texture(s, mi.normal_texture_index, uv);
         const f3 map{mn.x * 255.0f / 127.0f - 128.0f / 127.0f, mn.y * 255.0f / 127.0f - 128.0f / 127.0f,
@@ -771,6 +799,16 @@ LH_DEV f3 resolve_pixel(const lh_scene& s, const lh_view& v, uint32_t x, uint32_
         nrm = normalize3(f3{(t.x * map.x + b.x * map.y) + nrm.x * map.z, (t.y * map.x + b.y * map.y) + nrm.y * map.z,
                             (t.z * map.x + b.z * map.y) + nrm.z * map.z});
     }
+    uint32_t cascade = 0;
+    const float shadow_sum = shadow_factor(v, mi, world.v, &cascade);
+    const Lod lod_b = lod_of(s, mi.base_color_texture_index, uv), lod_m = lod_of(s, mi.metallic_roughness_texture_index, uv);
+    if (prm.frozen)
+        reinterpret_cast<uint4*>(prm.frozen)[size_t(y) * v.width + x] = pack_frozen(shadow_sum, flip, lod_b, lod_m);
+    const f4 bc = sample_texture_lod(s, mi.base_color_texture_index, lod_b, uv);
+    const f3 base = mul(f3{bc.x, bc.y, bc.z}, param_base_color(prm, mi, sf.mesh_info));
+    const f4 mr = sample_texture_lod(s, mi.metallic_roughness_texture_index, lod_m, uv);
+    const float roughness = mr.y * param_roughness(prm, s, sf.mesh_info);
+    const float metallic = mr.z * param_metallic(prm, s, sf.mesh_info);
     // Debug views (render_geometry.comp:268-308).
     switch (u.debug) {
         case UNIFORMS_DEBUG_CASCADES: return mul(base, debug_colour(cascade));
