@@ -27,8 +27,8 @@ lhd::OneView one(const lh_view* v) { return lhd::OneView{*v}; }
 
 namespace lhk {
 
-hipError_t raster_main(const lh_scene& s, const lhd::OneView& vs, const Tuning& t, hipStream_t st) {
-    hipError_t e = raster(s, vs, 0, 1, t.raster, st);
+hipError_t raster_main(const lh_scene& s, const lhd::OneView& vs, const Tuning& t, hipStream_t st, bool bins_clear) {
+    hipError_t e = raster(s, vs, 0, 1, t.raster, st, false, bins_clear);
     if (e == hipSuccess && (vs.v.flags & LH_VIEW_HIZ)) {
         e = hiz_cull(s, vs, t.cull_blocks, st);
         if (e == hipSuccess) e = raster(s, vs, 0, 1, t.raster, st, true);
@@ -41,12 +41,13 @@ hipError_t record_frame(const lh_scene& s, const lh_view& v, hipStream_t st) {
     const lhd::OneView vs{v};
     const uint64_t px = uint64_t(v.width) * v.height;
     // The attachment clears (src/rendering.cpp:206-211, :384) ride on the
-    // meshlet culls: the view's cull clears the visibility buffer, the
-    // cascades' cull the shadow maps, each before the raster that writes them.
+    // meshlet culls: the view's cull clears the visibility buffer (and the
+    // tiled raster's counts), the cascades' cull the shadow maps, each before the raster that writes them.
     hipError_t e = view_reset(vs, st);
     if (e == hipSuccess) e = cull_instances(s, vs, false, st);
-    if (e == hipSuccess) e = cull_meshlets(s, vs, 0, 1, tuning_for(v).cull_blocks, st, kClearVisbuffer);
-    if (e == hipSuccess) e = raster_main(s, vs, tuning_for(v), st);
+    const uint32_t bins = v.bin_capacity > 0 ? kClearBins : 0u;
+    if (e == hipSuccess) e = cull_meshlets(s, vs, 0, 1, tuning_for(v).cull_blocks, st, kClearVisbuffer | bins);
+    if (e == hipSuccess) e = raster_main(s, vs, tuning_for(v), st, bins != 0);
     if (e == hipSuccess) e = depth_bounds(vs, px, st);
     if (e == hipSuccess) e = fit_cull_instances_shadow(s, vs, st);
     if (e == hipSuccess) e = cull_meshlets(s, vs, 1, LH_NUM_CASCADES, tuning_for(v).cull_blocks, st, kClearShadowMaps);

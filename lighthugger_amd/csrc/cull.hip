@@ -20,6 +20,7 @@
 #include "hiz.h"
 #include "kernels.h"
 #include "lh_device.h"
+#include "scratch.h"
 
 using namespace lhd;
 
@@ -315,8 +316,14 @@ __global__ void __launch_bounds__(kCullThreads) k_cull_meshlets(lh_scene s, VS v
     }
     if (clear != 0) {
         const uint64_t b = uint64_t(blockIdx.y) * gridDim.x + blockIdx.x;
-        clear_part(v, (clear & lhk::kClearVisbuffer) != 0, (clear & lhk::kClearShadowMaps) != 0,
-                   b * blockDim.x + threadIdx.x, uint64_t(gridDim.x) * gridDim.y * blockDim.x);
+        const uint64_t t0 = b * blockDim.x + threadIdx.x, threads = uint64_t(gridDim.x) * gridDim.y * blockDim.x;
+        clear_part(v, (clear & lhk::kClearVisbuffer) != 0, (clear & lhk::kClearShadowMaps) != 0, t0, threads);
+        if (clear & lhk::kClearBins) {  // the tiled raster's tile counts and cursors
+            const lhs::ScratchLayout L = lhs::scratch_layout(v);
+            uint32_t* count = reinterpret_cast<uint32_t*>(static_cast<char*>(v.scratch) + L.tile_count);
+            uint32_t* cursor = reinterpret_cast<uint32_t*>(static_cast<char*>(v.scratch) + L.tile_cursor);
+            for (uint64_t t = t0; t < lhs::tile_words(L.tiles); t += threads) count[t] = cursor[t] = 0;
+        }
     }
 }
 

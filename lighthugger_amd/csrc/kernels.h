@@ -63,7 +63,7 @@ hipError_t fit_cull_instances_shadow(const lh_scene& s, const VS& vs, hipStream_
 // Render targets a meshlet-cull launch clears after its culling (the frame's
 // clears, moved into the latency-bound cull launches that precede the
 // rasters writing those targets).
-constexpr uint32_t kClearVisbuffer = 1, kClearShadowMaps = 2;
+constexpr uint32_t kClearVisbuffer = 1, kClearShadowMaps = 2, kClearBins = 4;  // kClearBins: the tile counts
 template <class VS>
 hipError_t cull_meshlets(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npasses, uint32_t blocks,
                          hipStream_t st, uint32_t clear = 0);
@@ -71,7 +71,7 @@ hipError_t cull_meshlets(const lh_scene& s, const VS& vs, uint32_t pass0, uint32
 // view alone, or any run of cascades).
 template <class VS>
 hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npasses, const RasterTuning& t,
-                  hipStream_t st, bool phase2 = false);
+                  hipStream_t st, bool phase2 = false, bool bins_clear = false);
 // LH_VIEW_HIZ: depth pyramid of the phase-1 raster and the occlusion test of
 // the staged candidates (appended to draws[0] for the phase-2 raster).
 hipError_t hiz_cull(const lh_scene& s, const lhd::OneView& vs, uint32_t blocks, hipStream_t st);
@@ -79,7 +79,9 @@ hipError_t hiz_cull(const lh_scene& s, const lhd::OneView& vs, uint32_t blocks, 
 hipError_t update_history(const lh_scene& s, const lhd::OneView& vs, hipStream_t st);
 // The main-view raster of one view: phase 1, and with LH_VIEW_HIZ the
 // pyramid, the occlusion test and phase 2.
-hipError_t raster_main(const lh_scene& s, const lhd::OneView& vs, const Tuning& t, hipStream_t st);
+// bins_clear: the meshlet cull before it zeroed the tile counts (kClearBins).
+hipError_t raster_main(const lh_scene& s, const lhd::OneView& vs, const Tuning& t, hipStream_t st,
+                       bool bins_clear = false);
 template <class VS>
 hipError_t depth_bounds(const VS& vs, uint64_t max_pixels, hipStream_t st);
 template <class VS>

@@ -165,17 +165,16 @@ LH_DEV float wave_sum_f32(float v) {
     });
     return __int_as_float(__builtin_amdgcn_readlane(s, 63));
 }
-LH_DEV uint32_t wave_sum_u32(uint32_t v) {
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
-}
+// Reductions over the wave, returned to every lane: the scans leave them in
+// lane 63.  The wave must be converged.
+LH_DEV uint32_t wave_sum_u32(uint32_t v) { return uint32_t(__builtin_amdgcn_readlane(int(wave_scan_add(v)), 63)); }
 LH_DEV uint32_t wave_min_u32(uint32_t v) {
-    for (int d = 32; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
-    return v;
+    const int32_t m = wave_scan_dpp(int32_t(v), -1, [](int32_t a, int32_t b) { return int32_t(min(uint32_t(a), uint32_t(b))); });
+    return uint32_t(__builtin_amdgcn_readlane(m, 63));
 }
 LH_DEV uint32_t wave_max_u32(uint32_t v) {
-    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    return v;
+    const int32_t m = wave_scan_dpp(int32_t(v), 0, [](int32_t a, int32_t b) { return int32_t(max(uint32_t(a), uint32_t(b))); });
+    return uint32_t(__builtin_amdgcn_readlane(m, 63));
 }
 
 // Wave-aggregated atomicAdd: returns the slot of each active lane with

@@ -49,8 +49,8 @@ struct PassSet {
     int32_t small_extent;   // subpixels: the tiled raster's in-lane boxes, up to this side
     int32_t medium_extent;  // subpixels: larger triangles go to the large-triangle queue (<= 64 px)
     uint32_t phase2;        // main view, second occlusion phase: draws from LH_CNT_HIZ_PHASE1 on
-    uint32_t direct;        // single view: rasterize only the draws the tiled raster left on its direct
-                            // list (flattened index | kBinDirect when their clip triangles are queued)
+    uint32_t direct;        // single view: rasterize the draws the tiled raster left on its direct list
+                            // (flattened index | kBinDirect when their queue triangles are queued already)
 };
 
 template <int KIND>
@@ -438,6 +438,30 @@ LH_DEV TriSetup triangle_setup(const WaveVerts& wv, uint32_t corners, bool live,
     return t;
 }
 
+// Appends to the clip and large-triangle queues (wave-aggregated; called by
+// the whole wave).
+LH_DEV void queue_clip(const lh_view& v, uint32_t pass0, bool pred, uint32_t d, uint32_t t, uint32_t pi, bool alpha) {
+    if (ballot(pred) == 0) return;
+    const uint32_t slot = wave_append(&v.counters[LH_CNT_CLIP + pass0], pred);
+    if (!pred) return;
+    if (slot < v.clip_capacity)
+        queues(v).clip[slot] = make_uint2((d << LH_KEY_TRI_BITS) | t, pi | (alpha ? kClipAlpha : 0u));
+    else
+        atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
+}
+LH_DEV void queue_big(const lh_view& v, uint32_t pass0, bool pred, const WaveVerts& wv, const TriSetup& ts, uint32_t id,
+                      uint32_t pi, bool alpha) {
+    if (ballot(pred) == 0) return;
+    const uint32_t slot = wave_append(&v.counters[LH_CNT_BIG + pass0], pred);
+    if (!pred) return;
+    const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]}, v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
+    if (slot < v.big_capacity)
+        store_big(queues(v).big + slot, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id, ts.xlo, ts.xhi, ts.ylo,
+                  ts.yhi, pi, alpha);
+    else
+        atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
+}
+
 // Triangles of up to kNarrow that are ready to be rasterized, collected over a
 // wave's meshlets.  Most set-up triangles of a dense scene cover no pixel
 // centre (4 of 64 do in the cascades of the 2,000-instance field), so the
@@ -458,6 +482,10 @@ struct TriQueueOf {
         };
         box[k] = make_uint4(uint32_t(xlo) | uint32_t(ylo) << 16, rel(v0), rel(v1), rel(v2));
         att[k] = make_uint4(__float_as_uint(v0.z), __float_as_uint(v1.z), __float_as_uint(v2.z), id);
+    }
+    LH_DEV void store(uint32_t k, const WaveVerts& wv, const TriSetup& ts, uint32_t id) {
+        const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]}, v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
+        store(k, ts.xlo, ts.ylo, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id);
     }
 };
 using TriQueue = TriQueueOf<kQueue>;
@@ -713,10 +741,10 @@ struct Segments<ViewTable> {
 }  // namespace lhr
 
 namespace lhk {
-// LDS-binned tiled raster of the main view (tile.hip): binning, scan, fill and
-// the tile kernel; the caller then runs the per-meshlet raster over the
-// direct list (PassSet::direct) and the clip / large-triangle launches.
+// LDS-binned tiled raster of the main view (tile.hip): binning, fill and the
+// tile kernel; the caller then draws the direct list (PassSet::direct) and the
+// queues.  bins_clear: the view's meshlet cull zeroed the tile counts.
 template <bool ST>
 hipError_t raster_tiles(const lh_scene& s, const lhd::OneView& vs, const lhr::PassSet& ps, const RasterTuning& t,
-                        hipStream_t st);
+                        bool bins_clear, hipStream_t st);
 }  // namespace lhk

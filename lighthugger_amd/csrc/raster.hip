@@ -51,17 +51,6 @@ namespace {
 #define LH_MESHLET_WAVES 6
 #endif
 
-// Queues of the clip and large-triangle kernels.
-LH_DEV void queue_clip(const lh_view& v, uint32_t pass0, bool pred, uint32_t d, uint32_t t, uint32_t pi, bool alpha) {
-    if (ballot(pred) == 0) return;
-    const uint32_t slot = wave_append(&v.counters[LH_CNT_CLIP + pass0], pred);
-    if (!pred) return;
-    if (slot < v.clip_capacity)
-        queues(v).clip[slot] = make_uint2((d << LH_KEY_TRI_BITS) | t, pi | (alpha ? kClipAlpha : 0u));
-    else
-        atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
-}
-
 // ALPHA selects the draws of alpha-clip mesh infos (double-sided, alpha test
 // per sample); the opaque instantiation skips them.  The alpha instantiation
 // returns at once when the culls counted no alpha-clip draw in its passes.
@@ -109,18 +98,18 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
         if (some == 0) break;
         DrawHead head{};
         uint32_t where = 0, draw = 0;
-        bool clip_queued = false;
+        bool binned = false;
         if (g < total) {
             const uint32_t e = list ? list[g] : g;
             uint32_t view, pi;
             seg.find(e & ~(list ? lhs::kBinDirect : 0u), view, pi, draw);
-            clip_queued = list && (e & lhs::kBinDirect) != 0;
+            binned = list && (e & lhs::kBinDirect) != 0;
             where = view << 3 | pi;
             const lh_view& v = vs.get(view);
             head = load_head(s, v.draws[size_t(ps.pass0 + pi) * v.draw_capacity + draw]);
         }
         uint64_t todo = ballot(g < total && (((head.info >> 16) & MESH_INFO_FLAGS_ALPHA_CLIP) != 0) == ALPHA);
-        const uint64_t clip_done = ballot(clip_queued);
+        const uint64_t queues_done = ballot(binned);
         if (todo == 0) continue;
         MeshletFetch next;
         DrawHead h = head_of_lane(head, first_lane(todo));
@@ -150,32 +139,17 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
             lds_order();
             if (todo) next.request_position(h, lane);
             const uint32_t ntri = cur.triangles();
+            const bool queued = ((queues_done >> l) & 1) != 0;  // by the tiled raster's binning
             for (uint32_t round = 0; round * 64 < ntri; round++) {
                 const uint32_t t = lane + 64 * round;
                 const TriSetup ts = triangle_setup<KIND>(wv, f.corners(cur, lane, round), t < ntri, clean, ALPHA, p.W, p.H);
-                if (!clean && !((clip_done >> l) & 1)) queue_clip(v, ps.pass0, ts.clip, d, t, pi, ALPHA);
+                if (!clean) queue_clip(v, ps.pass0, ts.clip && !queued, d, t, pi, ALPHA);
                 const bool big = ts.inside && ts.extent > ps.medium_extent, push = ts.inside && !big;
                 const uint32_t id = (cur.mid << LH_KEY_TRI_BITS) | t;
-                if (ballot(big)) {
-                    const uint32_t slot = wave_append(&v.counters[LH_CNT_BIG + ps.pass0], big);
-                    if (big) {
-                        const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]},
-                            v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
-                        if (slot < v.big_capacity)
-                            store_big(queues(v).big + slot, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id, ts.xlo,
-                                      ts.xhi, ts.ylo, ts.yhi, pi, ALPHA);
-                        else
-                            atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
-                    }
-                }
+                queue_big(v, ps.pass0, big && !queued, wv, ts, id, pi, ALPHA);
                 const uint64_t pm = ballot(push);
                 if (pm == 0) continue;
-                if (push) {
-                    const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]},
-                        v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
-                    queue.store(held + lanes_below(pm), ts.xlo, ts.ylo, v0, ts.swapped ? v2 : v1,
-                                ts.swapped ? v1 : v2, id);
-                }
+                if (push) queue.store(held + lanes_below(pm), wv, ts, id);
                 held += uint32_t(__popcll(pm));
                 if (held >= 64) {  // the last 64 entries: nothing moves
                     held -= 64;
@@ -358,6 +332,41 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
     // the queue are neighbours on a mesh and of much the same size, so a
     // wave's entries lie `waves` apart: a run of large ones is shared out.
     const uint32_t waves = gridDim.x * 4;
+    // The draws that the tiled raster left because of their size (few): their
+    // triangles within the medium extent; the others are queued already.
+    if constexpr (KIND == 0 && !ALPHA && std::is_same<VS, OneView>::value) {
+        __shared__ WaveVerts verts4[4];
+        WaveVerts& wv = verts4[wave];
+        const lhs::ScratchLayout L = lhs::scratch_layout(v);
+        const uint32_t* list = reinterpret_cast<const uint32_t*>(static_cast<const char*>(v.scratch) + L.direct);
+        const uint32_t n = ps.direct ? min(v.counters[LH_CNT_TILE_DIRECT], L.direct_capacity) : 0u;
+        const Segments<VS> seg(vs, ps);
+        const Pass p = make_pass(v, ps.pass0);
+        for (uint32_t i = blockIdx.x * 4 + wave; i < n; i += waves) {
+            uint32_t view, pi, d;
+            seg.find(uniform_u32(list[i]) & ~lhs::kBinDirect, view, pi, d);
+            const DrawHead h = head_of_lane(load_head(s, p.draws[d]), 0);
+            MeshletFetch f;
+            f.request(h, lane);
+            f.request_position(h, lane);
+            const LhMat4 T = load_mat4(reinterpret_cast<uint64_t>(&s.instances[h.instance].transform));
+            const LhMat4 M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
+            SV sv;
+            lds_order();
+            const bool clean = transform_vertices(h, f, T, M, p.W, p.H, lane, wv, sv);
+            lds_order();
+            for (uint32_t r = 0; r * 64 < h.triangles(); r++) {
+                const uint32_t t = lane + 64 * r;
+                const TriSetup ts =
+                    triangle_setup<KIND>(wv, f.corners(h, lane, r), t < h.triangles(), clean, false, p.W, p.H);
+                const bool push = ts.inside && ts.extent <= ps.medium_extent;
+                const uint64_t pm = ballot(push);
+                if (pm == 0) continue;
+                if (push) queue.store(lanes_below(pm), wv, ts, (h.mid << LH_KEY_TRI_BITS) | t);
+                raster_narrow(uint32_t(__popcll(pm)), p);
+            }
+        }
+    }
     auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + blockIdx.x * 4 + w + l * waves; };
     uint32_t round = 0;
     for (uint32_t b0 = 0; b0 + blockIdx.x * 4 < count; b0 += 64 * waves, round ^= 1) {  // block-uniform
@@ -482,29 +491,32 @@ namespace lhk {
 // covers only the draws it left.
 template <int KIND, bool ST, class VS>
 hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const RasterTuning& t, uint32_t big_blocks,
-                          hipStream_t st) {
+                          bool bins_clear, hipStream_t st) {
     const uint32_t nv = vs.count();
     bool tiled = false;
     if constexpr (std::is_same<VS, OneView>::value)
         tiled = KIND == 0 && vs.v.bin_capacity > 0 && t.tile_raster != 0;
-    if (tiled) {
-        if constexpr (std::is_same<VS, OneView>::value) {
-            hipError_t e = raster_tiles<ST>(s, vs, ps, t, st);
-            if (e != hipSuccess) return e;
-        }
-        ps.direct = 1;
-        mark("raster_direct_view", st);
-    } else {
-        mark(KIND == 0 ? "raster_meshlets_view" : "raster_meshlets_shadow", st);
-    }
     // The draw count is on the device; the scene's meshlets bound what a pass
     // can draw (a block without a draw still costs its launch: 24,576 empty
-    // ones 4 us).  The direct list is short or empty.
+    // ones 4 us).
     const uint64_t most = uint64_t(std::max(s.total_meshlets, 1u)) * nv;
     const uint32_t blocks = uint32_t(std::min<uint64_t>(t.meshlet_blocks, most));
-    hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST>), dim3(tiled ? std::min(blocks, 1024u) : blocks), dim3(64), 0,
-                       st, s, vs, ps);
-    ps.direct = 0;
+    bool direct = false;  // the direct list is drawn by the large-triangle launch
+    if (tiled) {
+        if constexpr (std::is_same<VS, OneView>::value) {
+            hipError_t e = raster_tiles<ST>(s, vs, ps, t, bins_clear, st);
+            if (e != hipSuccess) return e;
+            // every draw can be binned: the list holds only the few that are
+            // too large for the bins; else any number beyond the bins
+            direct = vs.v.bin_capacity >= std::min(vs.v.draw_capacity, s.total_meshlets);
+        }
+    }
+    if (!tiled || !direct) {
+        ps.direct = tiled ? 1u : 0u;
+        mark(tiled ? "raster_direct_view" : KIND == 0 ? "raster_meshlets_view" : "raster_meshlets_shadow", st);
+        hipLaunchKernelGGL((k_raster_meshlets<KIND, VS, ST>), dim3(blocks), dim3(64), 0, st, s, vs, ps);
+        ps.direct = 0;
+    }
     const bool alpha = !(s.flags & LH_SCENE_OPAQUE_ONLY);
     if (alpha) {
         mark(KIND == 0 ? "raster_alpha_view" : "raster_alpha_shadow", st);
@@ -512,6 +524,7 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
         pa.medium_extent = std::min(ps.medium_extent, kAlphaMediumPx * 256);
         hipLaunchKernelGGL((k_raster_alpha<KIND, VS, ST>), dim3(blocks), dim3(64), 0, st, s, vs, pa);
     }
+    ps.direct = direct ? 1u : 0u;
     mark(KIND == 0 ? "raster_big_view" : "raster_big_shadow", st);
     hipLaunchKernelGGL((k_raster_big<KIND, VS, ST, false>), dim3(big_blocks, 1, nv), dim3(256), 0, st, s, vs, ps);
     if (alpha) {
@@ -524,19 +537,19 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
 // Statistics are a single-view feature (LH_VIEW_STATISTICS).
 template <int KIND>
 hipError_t launch_set(const lh_scene& s, const OneView& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
-                      hipStream_t st) {
-    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, bb, st);
-    return launch_kernels<KIND, false>(s, vs, ps, t, bb, st);
+                      bool bins_clear, hipStream_t st) {
+    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, bb, bins_clear, st);
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, bins_clear, st);
 }
 template <int KIND>
 hipError_t launch_set(const lh_scene& s, const ViewTable& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
-                      hipStream_t st) {
-    return launch_kernels<KIND, false>(s, vs, ps, t, bb, st);
+                      bool bins_clear, hipStream_t st) {
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, bins_clear, st);
 }
 
 template <class VS>
 hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npasses, const RasterTuning& t,
-                  hipStream_t st, bool phase2) {
+                  hipStream_t st, bool phase2, bool bins_clear) {
     if (npasses == 0 || npasses > LH_NUM_CASCADES || pass0 + npasses > LH_NUM_PASSES || (pass0 == 0 && npasses != 1))
         return hipErrorInvalidValue;
     // the cascades may take their own extents (their triangles are smaller
@@ -550,14 +563,14 @@ hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npas
     const uint32_t nv = vs.count();
     // the per-view persistent grid of the queue kernel shrinks with the batch size
     const uint32_t big_blocks = nv > 1 ? std::max(t.big_blocks / 16, 32u) : t.big_blocks;
-    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, big_blocks, st);
-    return launch_set<1>(s, vs, ps, t, big_blocks, st);
+    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, big_blocks, bins_clear, st);
+    return launch_set<1>(s, vs, ps, t, big_blocks, bins_clear, st);
 }
 
 template hipError_t raster<OneView>(const lh_scene&, const OneView&, uint32_t, uint32_t, const RasterTuning&,
-                                    hipStream_t, bool);
+                                    hipStream_t, bool, bool);
 template hipError_t raster<ViewTable>(const lh_scene&, const ViewTable&, uint32_t, uint32_t, const RasterTuning&,
-                                      hipStream_t, bool);
+                                      hipStream_t, bool, bool);
 
 hipError_t plan_segments(const ViewTable& vt, uint32_t pass0, uint32_t npasses, hipStream_t st) {
     if (vt.n * npasses > LH_MAX_BATCH_SEGMENTS) return hipErrorInvalidValue;

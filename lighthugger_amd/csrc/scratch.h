@@ -57,6 +57,8 @@ struct ScratchLayout {
 };
 
 LH_HD uint64_t align256(uint64_t n) { return (n + 255) & ~uint64_t(255); }
+// Words of the tile count and cursor arrays in use: whole 64-byte lines.
+LH_HD uint32_t tile_words(uint32_t tiles) { return (tiles + 15) & ~15u; }
 
 LH_HD ScratchLayout scratch_layout(uint32_t width, uint32_t height, uint32_t draw_capacity, uint32_t big_capacity,
                                    uint32_t clip_capacity, uint32_t bin_capacity) {

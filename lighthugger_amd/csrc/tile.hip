@@ -16,22 +16,20 @@
 //                   pixel bounding boxes to the bin header; clip-crossing
 //                   triangles to the clip queue and triangles over the medium
 //                   extent to the large-triangle queue, as in the per-meshlet
-//                   raster.
-//   k_bin_count     one thread per draw: reserves its (meshlet, tile) entries,
-//                   counts them per tile; draws that cannot be binned (over
-//                   bin_capacity, too many tiles, no entry left) go to the
-//                   direct list for the per-meshlet raster.
-//   k_bin_scan      one block: tile offsets and work items of at most
-//                   `item_entries` entries per tile.
-//   k_bin_fill      one thread per draw: writes its entries.
+//                   raster.  The meshlet's tiles are counted; draws that
+//                   cannot be binned (over bin_capacity, too many tiles) go to
+//                   the direct list.
+//   k_bin_fill      tile offsets, work items of at most `item_entries` entries
+//                   per tile, and the (draw, part) entries.
 //   k_tile_raster   persistent blocks of 8 waves over the items: LDS tile
 //                   cleared, each wave rasterizes one binned meshlet at a time
 //                   (two when their triangles fit one round) from the cache
 //                   (ds_min_u64 per covered sample), then the tile's covered
 //                   pixels are written out.
-// The per-meshlet raster then runs over the direct list, followed by the
-// alpha-clip, clip and large-triangle launches (all device-scope atomicMin on
-// top of what the tiles wrote).
+// The direct list is then drawn by the large-triangle launch (or, when the
+// caller's bin_capacity is below its draw capacity, by the per-meshlet raster),
+// followed by the alpha-clip launches (all device-scope atomicMin on top of
+// what the tiles wrote).
 #include "raster.h"
 
 using namespace lhd;
@@ -46,7 +44,6 @@ namespace {
 constexpr uint32_t kTile = LH_TILE_SIDE;
 constexpr uint32_t kTileWaves = 8;
 constexpr uint32_t kTileThreads = 64 * kTileWaves;
-constexpr uint32_t kScanThreads = 1024;
 
 struct Bins {
     BinHeader* hdr;
@@ -71,8 +68,14 @@ LH_DEV Bins bins(const lh_view& v) {
             L};
 }
 
-LH_DEV uint32_t rect_tiles(uint32_t r) {
-    return (((r >> 16) & 255u) - (r & 255u) + 1u) * ((r >> 24) - ((r >> 8) & 255u) + 1u);
+// Word of tile t in the count and cursor arrays.  Device atomics to one cache
+// line serialize as those to one word do, and the busy tiles of a view are
+// neighbours (the horizon's row): consecutive tiles lie in different 64-byte
+// lines.  (Binning the 20,000-instance field at 4K: 1.71 ms with the tiles in
+// order.)  The arrays end on a 256-byte boundary, so the last line is whole.
+LH_DEV uint32_t tile_word(uint32_t t, uint32_t tiles) {
+    const uint32_t lines = (tiles + 15) / 16;
+    return (t % lines) * 16 + t / lines;
 }
 
 // Draws [0, n) of the launch binned by k_bin_meshlets.
@@ -80,150 +83,152 @@ LH_DEV uint32_t binned_draws(const Segments<OneView>& seg, const lh_view& v) { r
 
 // ---------------------------------------------------------------- binning
 
-// One wave per draw g < min(total, bin_capacity).  Alpha-clip meshlets are
-// left to the alpha-clip raster (header with no triangles).
-template <int KIND>
-__global__ void __launch_bounds__(64) LH_RASTER_OCCUPANCY k_bin_meshlets(lh_scene s, OneView vs, PassSet ps) {
-    __shared__ int32_t sX[64], sY[64];
-    __shared__ float sZ[64];
-    __shared__ uint32_t sO[64];
-    const uint32_t lane = threadIdx.x;
-    const lh_view& v = vs.v;
-    const Segments<OneView> seg(vs, ps);
-    const uint32_t total = binned_draws(seg, v);
-    const Bins B = bins(v);
-    const Queues qs = queues(v);
-    uint32_t* clip_counter = &v.counters[LH_CNT_CLIP + ps.pass0];
-    uint32_t* big_counter = &v.counters[LH_CNT_BIG + ps.pass0];
-    // this launch's tile counts and reservations start from zero (k_bin_count runs after it)
-    for (uint32_t t = blockIdx.x * 64 + lane; t < B.L.tiles; t += gridDim.x * 64) B.tile_count[t] = 0;
-    if (blockIdx.x == 0 && lane == 0) {
-        v.counters[LH_CNT_TILE_DIRECT] = 0;
-        v.counters[LH_CNT_TILE_ITEMS] = 0;
-    }
-    for (uint32_t g = blockIdx.x; g < total; g += gridDim.x) {
-        uint32_t view, pi, d;
-        seg.find(g, view, pi, d);
-        const Pass p = make_pass(v, ps.pass0 + pi);
-        const LhMat4& M = view_matrix<KIND>(v, p.pass);
-        const MeshletReference ref = p.draws[d];
-        const Instance& in = s.instances[ref.instance_index];
-        const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
-        const uint32_t mid = s.instance_meshlet_base[ref.instance_index] + ref.meshlet_index;
-        if (mi.flags & MESH_INFO_FLAGS_ALPHA_CLIP) {  // wave-uniform
-            if (lane == 0) B.hdr[g] = BinHeader{0u, 0u, mid, 0u};
-            continue;
-        }
-        const Meshlet& ml = ptr<Meshlet>(mi.meshlets)[ref.meshlet_index];
-        const uint32_t nvert = ml.index_count, ntri = ml.triangle_count;
-        const uint8_t* micro = ptr<uint8_t>(mi.micro_indices) + ml.triangle_offset;
-        uint32_t corners[2] = {0u, 0u};
-        for (uint32_t r = 0; r < 2; r++) {
-            const uint32_t t = lane + 64 * r;
-            if (t < ntri)
-                corners[r] = uint32_t(micro[3 * t]) | (uint32_t(micro[3 * t + 1]) << 8) |
-                             (uint32_t(micro[3 * t + 2]) << 16);
-        }
-        BinCache& c = B.cache[g];
-        if (lane < nvert) {
-            f3 w = mat4_point(in.transform, load_position(mi, load_index(mi, ml.index_offset + lane)));
-            f4 q = mat4_mul_vec4(M, f4{w.x, w.y, w.z, 1.0f});
-            uint32_t oc = finite4(q) ? outcode(q) : kBadVertex;
-            SV sv{0, 0, 0.0f};
-            if (oc == 0 && !project(q, p.W, p.H, sv)) oc = kBadVertex;
-            sX[lane] = sv.X;
-            sY[lane] = sv.Y;
-            sZ[lane] = sv.z;
-            sO[lane] = oc;
-            c.X[lane] = sv.X;
-            c.Y[lane] = sv.Y;
-            c.Z[lane] = sv.z;
-        }
-        __syncthreads();
-        int32_t xlo_m = 0x7FFFFFFF, ylo_m = 0x7FFFFFFF, xhi_m = -1, yhi_m = -1;
-        uint32_t nfront = 0, work = 0;  // work: pixels of the front triangles' boxes
-        for (uint32_t round = 0; round < 2; round++) {
-            const uint32_t t = lane + 64 * round;
-            if (__ballot(t < ntri) == 0) break;
-            // Every lane sets up its triangle (lanes past the meshlet read
-            // corner 0 three times: zero area; clipped corners read as zero)
-            // and the outcome is flat predicates, not nested branches whose
-            // exits would each re-zero the setup's registers.
-            uint32_t packed = corners[round];
-            const uint32_t i0 = packed & 255u, i1 = (packed >> 8) & 255u, i2 = packed >> 16;
-            const uint32_t o0 = sO[i0], o1 = sO[i1], o2 = sO[i2];
-            SV v0{sX[i0], sY[i0], sZ[i0]}, v1{sX[i1], sY[i1], sZ[i1]}, v2{sX[i2], sY[i2], sZ[i2]};
-            int64_t area;
-            int32_t xlo, xhi, ylo, yhi, ex, ey;
-            bool swapped;
-            const bool set = setup<KIND>(v0, v1, v2, p.W, p.H, area, xlo, xhi, ylo, yhi, ex, ey, false, &swapped);
-            const bool drawn = t < ntri && ((o0 | o1 | o2) & kBadVertex) == 0 && (o0 & o1 & o2) == 0;
-            const bool clip = drawn && (o0 | o1 | o2) != 0;
-            const bool inside = drawn && (o0 | o1 | o2) == 0 && set;
-            // triangles over the medium extent: spread over many blocks by the large-triangle raster
-            const bool big = inside && max(ex, ey) > ps.medium_extent;
-            const bool front = inside && !big;
-            if (front) {
-                if (swapped) packed = i0 | (i2 << 8) | (i1 << 16);
-                xlo_m = min(xlo_m, xlo);
-                ylo_m = min(ylo_m, ylo);
-                xhi_m = max(xhi_m, xhi);
-                yhi_m = max(yhi_m, yhi);
-                work += uint32_t((xhi - xlo + 1) * (yhi - ylo + 1));
-            }
-            const uint32_t cslot = wave_append(clip_counter, clip);
-            if (clip) {
-                if (cslot < v.clip_capacity)
-                    qs.clip[cslot] = make_uint2((d << LH_KEY_TRI_BITS) | t, pi);
-                else
-                    atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
-            }
-            const uint32_t bslot = wave_append(big_counter, big);
-            if (big) {
-                if (bslot < v.big_capacity)
-                    store_big(qs.big + bslot, v0, v1, v2, (mid << LH_KEY_TRI_BITS) | t, xlo, xhi, ylo, yhi, pi, false);
-                else
-                    atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
-            }
-            const uint64_t fm = ballot(front);
-            if (front) c.tri[nfront + lanes_below(fm)] = packed | (t << 24);
-            nfront += uint32_t(__popcll(fm));
-        }
-        const int32_t x0 = int32_t(wave_min_u32(uint32_t(xlo_m))), y0 = int32_t(wave_min_u32(uint32_t(ylo_m)));
-        const int32_t x1 = int32_t(wave_max_u32(uint32_t(xhi_m + 1))) - 1,
-                      y1 = int32_t(wave_max_u32(uint32_t(yhi_m + 1))) - 1;
-        const uint32_t total_work = wave_sum_u32(work);
-        if (lane == 0) {
-            BinHeader h{0u, 0u, mid, 0u};
-            if (nfront) {
-                h.rect = (uint32_t(x0) >> lhs::kTileShift) | ((uint32_t(y0) >> lhs::kTileShift) << 8) |
-                         ((uint32_t(x1) >> lhs::kTileShift) << 16) | ((uint32_t(y1) >> lhs::kTileShift) << 24);
-                // a meshlet with much pixel work is split by triangle range into 2^lp parts, each its own
-                // entry (so its work spreads over several waves), within LH_TILE_MAX_RECT entries in all
-                const uint32_t tiles = rect_tiles(h.rect);
-                uint32_t lp = 0;
-                while (lp < lhs::kMaxPartsLog2 && (total_work >> (lhs::kPartWorkLog2 + lp)) != 0 &&
-                       (tiles << (lp + 1)) <= LH_TILE_MAX_RECT && (nfront >> (lp + 1)) >= 8)
-                    lp++;
-                h.ntri = nfront | (lp << lhs::kPartShift);
-            }
-            B.hdr[g] = h;
-        }
-        __syncthreads();
+// Zeroes the tile counts and cursors and the counters of a main-view raster
+// that does not follow a meshlet cull which has done so (kClearBins).
+__global__ void __launch_bounds__(256) k_bin_reset(OneView vs) {
+    const Bins B = bins(vs.v);
+    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < lhs::tile_words(B.L.tiles); t += gridDim.x * 256)
+        B.tile_count[t] = B.tile_cursor[t] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        vs.v.counters[LH_CNT_TILE_DIRECT] = 0;
+        vs.v.counters[LH_CNT_TILE_ITEMS] = 0;
     }
 }
 
-// Per-tile counters are aggregated in LDS per block before they reach the
-// device (same-address device atomics serialize): a block handles runs of
-// kBinChunk consecutive draws and tiles up to kHistTiles; views with more
-// tiles count in device memory directly.  One draw per thread and chunk: the
-// grid is sized for the draw capacity, and longer chunks left most blocks
-// without a chunk when far fewer draws survive (the large frame: 66k draws,
-// 33 busy blocks at 2,048 draws a chunk; the fill pass took 0.024 ms, 0.011
-// at 256).
-constexpr uint32_t kBinThreads = 256;
-constexpr uint32_t kBinChunk = kBinThreads;
-constexpr uint32_t kHistTiles = 16384;  // 128 x 128 tiles: an 8192 x 8192 view
+// Occupancy (waves per SIMD), grid (two rounds of what is resident) and the
+// fewest draws per wave of the binning.  Bound by VALU issue (about 400
+// instructions a meshlet) and, with many large triangles, by the appends to
+// their queue.  500 k meshlets of the 20,000-instance field at 4K: 446 us one
+// draw at a time plus 15 for a launch that counted the tiles; 359, 311, 296 us
+// on 7,168, 14,336, 28,672 blocks at 7 waves, 330 at 6, 363 at 8.  The 1080p
+// field (59 k): 60 + 8 -> 53 us; 56 and 60 with at least 8 and 12 draws.
+#define LH_BIN_WAVES 7
+constexpr uint32_t kBinBlocks = 14336;
+constexpr uint32_t kBinShare = 2;
+
+// One wave per draw g < min(total, bin_capacity); later draws go to the direct
+// list.  Alpha-clip meshlets are left to the alpha-clip raster (header with no
+// triangles).  The heads of a wave's next 64 draws are loaded together, and a
+// meshlet's vertices requested while the one before is in hand (as in the
+// meshlet raster).  A wave's draws are consecutive, so that they share most of
+// their tiles, and it adds their counts to the tiles' together: one atomic per
+// distinct tile (one per meshlet and tile took the binning of the 1080p field
+// from 55 to 82 us: same-address atomics serialize).
+template <int KIND>
+__global__ void __launch_bounds__(64) LH_WAVES_ATTR(LH_BIN_WAVES) k_bin_meshlets(lh_scene s, OneView vs, PassSet ps) {
+    __shared__ WaveVerts wv;
+    const uint32_t lane = threadIdx.x;
+    const lh_view& v = vs.v;
+    const Segments<OneView> seg(vs, ps);
+    const uint32_t all = seg.total(), total = binned_draws(seg, v);
+    const Bins B = bins(v);
+    const Pass p = make_pass(v, ps.pass0);
+    const LhMat4 M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
+    for (uint32_t g0 = total + blockIdx.x * 64; g0 < all; g0 += gridDim.x * 64) {
+        const uint32_t slot = wave_append(&v.counters[LH_CNT_TILE_DIRECT], g0 + lane < all);
+        if (g0 + lane < all && slot < B.L.direct_capacity) B.direct[slot] = g0 + lane;
+    }
+    const uint32_t share = max((total + gridDim.x - 1) / gridDim.x, kBinShare), last = min((blockIdx.x + 1) * share, total);
+    for (uint32_t k0 = blockIdx.x * share; k0 < last; k0 += 64) {
+        const uint32_t my_g = k0 + lane;
+        DrawHead head{};
+        uint32_t my_d = 0, my_rect = 0, my_tiles = 0, my_parts = 0;
+        if (my_g < last) {
+            uint32_t view, pi;
+            seg.find(my_g, view, pi, my_d);
+            head = load_head(s, p.draws[my_d]);
+            if (head.has(MESH_INFO_FLAGS_ALPHA_CLIP)) B.hdr[my_g] = BinHeader{0u, 0u, head.mid, 0u};
+        }
+        uint64_t todo = ballot(my_g < last && !head.has(MESH_INFO_FLAGS_ALPHA_CLIP));
+        if (todo == 0) continue;
+        MeshletFetch next;
+        DrawHead h = head_of_lane(head, first_lane(todo));
+        next.request(h, lane);
+        next.request_position(h, lane);
+        while (todo) {
+            const uint32_t l = first_lane(todo);
+            todo &= todo - 1;
+            const DrawHead cur = h;
+            MeshletFetch f = next;
+            if (todo) {
+                h = head_of_lane(head, first_lane(todo));
+                next.request(h, lane);
+            }
+            const uint32_t g = k0 + l, d = readlane_u32(my_d, l);
+            const LhMat4 T = load_mat4(reinterpret_cast<uint64_t>(&s.instances[cur.instance].transform));
+            SV sv;
+            lds_order();
+            const bool clean = transform_vertices(cur, f, T, M, p.W, p.H, lane, wv, sv);
+            lds_order();
+            BinCache& c = B.cache[g];
+            if (lane < cur.vertices()) {
+                c.X[lane] = sv.X;
+                c.Y[lane] = sv.Y;
+                c.Z[lane] = sv.z;
+            }
+            if (todo) next.request_position(h, lane);
+            const uint32_t ntri = cur.triangles();
+            int32_t xlo_m = 0x7FFFFFFF, ylo_m = 0x7FFFFFFF, xhi_m = -1, yhi_m = -1;
+            uint32_t nfront = 0, work = 0;  // work: pixels of the front triangles' boxes
+            for (uint32_t round = 0; round * 64 < ntri; round++) {
+                const uint32_t t = lane + 64 * round;
+                const TriSetup ts = triangle_setup<KIND>(wv, f.corners(cur, lane, round), t < ntri, clean, false, p.W, p.H);
+                if (!clean) queue_clip(v, ps.pass0, ts.clip, d, t, 0, false);
+                // triangles over the medium extent: spread over many blocks by the large-triangle raster
+                const bool big = ts.inside && ts.extent > ps.medium_extent, front = ts.inside && !big;
+                queue_big(v, ps.pass0, big, wv, ts, (cur.mid << LH_KEY_TRI_BITS) | t, 0, false);
+                const uint64_t fm = ballot(front);
+                if (front) {
+                    xlo_m = min(xlo_m, ts.xlo), ylo_m = min(ylo_m, ts.ylo);
+                    xhi_m = max(xhi_m, ts.xhi), yhi_m = max(yhi_m, ts.yhi);
+                    work += uint32_t(__mul24(ts.xhi - ts.xlo + 1, ts.yhi - ts.ylo + 1));
+                    const uint32_t b = ts.swapped ? ts.i2 : ts.i1, e = ts.swapped ? ts.i1 : ts.i2;
+                    c.tri[nfront + lanes_below(fm)] = ts.i0 | (b << 8) | (e << 16) | (t << 24);
+                }
+                nfront += uint32_t(__popcll(fm));
+            }
+            if (nfront == 0) {  // wave-uniform
+                if (lane == 0) B.hdr[g] = BinHeader{0u, 0u, cur.mid, 0u};
+                continue;
+            }
+            const uint32_t x0 = wave_min_u32(uint32_t(xlo_m)) >> lhs::kTileShift, y0 = wave_min_u32(uint32_t(ylo_m)) >> lhs::kTileShift;
+            const uint32_t x1 = (wave_max_u32(uint32_t(xhi_m + 1)) - 1) >> lhs::kTileShift,
+                           y1 = (wave_max_u32(uint32_t(yhi_m + 1)) - 1) >> lhs::kTileShift;
+            const uint32_t total_work = wave_sum_u32(work);
+            // a meshlet with much pixel work is split by triangle range into 2^lp parts, each its own
+            // entry (so its work spreads over several waves), within LH_TILE_MAX_RECT entries in all
+            const uint32_t nx = x1 - x0 + 1, tiles = nx * (y1 - y0 + 1);
+            uint32_t lp = 0;
+            while (lp < lhs::kMaxPartsLog2 && (total_work >> (lhs::kPartWorkLog2 + lp)) != 0 &&
+                   (tiles << (lp + 1)) <= LH_TILE_MAX_RECT && (nfront >> (lp + 1)) >= 8)
+                lp++;
+            // too many tiles: left to the per-meshlet path
+            const bool direct = tiles > LH_TILE_MAX_RECT;
+            const uint32_t rect = x0 | (y0 << 8) | (x1 << 16) | (y1 << 24);
+            if (lane == l) my_rect = rect, my_tiles = direct ? 0u : tiles, my_parts = 1u << lp;
+            if (lane == 0) {
+                B.hdr[g] = BinHeader{rect, nfront | (lp << lhs::kPartShift) | (direct ? lhs::kBinDirect : 0u), cur.mid, 0u};
+                if (direct) {
+                    const uint32_t slot = atomicAdd(&v.counters[LH_CNT_TILE_DIRECT], 1u);
+                    if (slot < B.L.direct_capacity) B.direct[slot] = g | lhs::kBinDirect;
+                }
+            }
+        }
+        // the i-th tiles of all the wave's meshlets, merged
+        uint32_t tx = my_rect & 255u, ty = (my_rect >> 8) & 255u;
+        for (uint32_t i = 0, most = wave_max_u32(my_tiles); i < most; i++) {
+            const uint32_t tile = ty * B.L.tiles_x + tx;
+            for (uint64_t left = ballot(i < my_tiles); left;) {
+                const uint32_t t = readlane_u32(tile, first_lane(left));
+                const bool mine = i < my_tiles && tile == t;
+                const uint32_t n = wave_sum_u32(mine ? my_parts : 0u);
+                if (lane == 0) atomicAdd(&B.tile_count[tile_word(t, B.L.tiles)], n);
+                left &= ~ballot(mine);
+            }
+            if (++tx > ((my_rect >> 16) & 255u)) tx = my_rect & 255u, ty++;
+        }
+    }
+}
 
 LH_DEV void for_each_tile(uint32_t rect, uint32_t tiles_x, auto&& f) {
     const uint32_t tx0 = rect & 255u, ty0 = (rect >> 8) & 255u, tx1 = (rect >> 16) & 255u, ty1 = rect >> 24;
@@ -231,115 +236,77 @@ LH_DEV void for_each_tile(uint32_t rect, uint32_t tiles_x, auto&& f) {
         for (uint32_t tx = tx0; tx <= tx1; tx++) f(ty * tiles_x + tx);
 }
 
-// One thread per draw of the launch.  Draws past bin_capacity and those whose
-// rectangle exceeds LH_TILE_MAX_RECT tiles go to the direct list (flattened
-// index, kBinDirect when k_bin_meshlets queued their clip triangles); the
-// entry list holds LH_TILE_MAX_RECT entries per binned draw, so every other
-// draw finds room.
-__global__ void __launch_bounds__(kBinThreads) k_bin_count(OneView vs, PassSet ps) {
-    __shared__ uint32_t hist[kHistTiles];
+// The entry lists and the work items.  Every block scans the tile counts into
+// entry and item offsets by itself (a few loads per thread, from the L2)
+// instead of waiting for a launch that would; the items, runs of at most
+// `item_entries` entries per tile, are shared out over the blocks tile by
+// tile.  Then one thread per binned draw puts its entries at the tiles'
+// cursors: per run of kBinThreads draws a block counts its entries per tile in
+// LDS, reserves each tile's range with one device atomic, and hands out the
+// slots in LDS (same-address device atomics serialize).  In views of more than
+// kHistTiles tiles the offsets fill the LDS: block 0 writes the items and every
+// slot comes from the device cursor.
+constexpr uint32_t kBinThreads = 256;
+constexpr uint32_t kHistTiles = 8192;
+constexpr uint32_t kMaxTiles = (LH_MAX_VIEW_SIDE / LH_TILE_SIDE) * (LH_MAX_VIEW_SIDE / LH_TILE_SIDE);
+static_assert(kMaxTiles <= 2 * kHistTiles, "the offsets of the largest view fit the shared array");
+__global__ void __launch_bounds__(kBinThreads) k_bin_fill(OneView vs, PassSet ps, uint32_t item_entries) {
+    __shared__ uint32_t shared[2 * kHistTiles];
+    __shared__ uint32_t wsum[2][kBinThreads / 64];
     const lh_view& v = vs.v;
     const Segments<OneView> seg(vs, ps);
-    const uint32_t total = seg.total();
     const uint32_t nb = binned_draws(seg, v);
     const Bins B = bins(v);
-    const bool lds = B.L.tiles <= kHistTiles;
-    if (lds)
-        for (uint32_t t = threadIdx.x; t < B.L.tiles; t += kBinThreads) hist[t] = 0;
-    __syncthreads();
-    for (uint32_t base = blockIdx.x * kBinThreads; base < total; base += gridDim.x * kBinThreads) {
-        const uint32_t g = base + threadIdx.x;
-        bool direct = false;
-        uint32_t rect = 0, n = 0, tag = 0, parts = 1;
-        if (g < nb) {
-            const BinHeader h = B.hdr[g];
-            if (h.ntri) {
-                rect = h.rect;
-                n = rect_tiles(rect);
-                parts = 1u << lhs::parts_log2(h.ntri);
-                if (n > LH_TILE_MAX_RECT) {
-                    direct = true;
-                    n = 0;
-                }
-                tag = lhs::kBinDirect;
-            }
-        } else if (g < total) {
-            direct = true;
-        }
-        if (direct && g < nb) B.hdr[g].ntri |= lhs::kBinDirect;
-        const uint32_t slot = wave_append(&v.counters[LH_CNT_TILE_DIRECT], direct);
-        if (direct && slot < B.L.direct_capacity) B.direct[slot] = g | tag;
-        if (n) {
-            if (lds)
-                for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) { atomicAdd(&hist[t], parts); });
-            else
-                for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) { atomicAdd(&B.tile_count[t], parts); });
-        }
-    }
-    __syncthreads();
-    if (lds)
-        for (uint32_t t = threadIdx.x; t < B.L.tiles; t += kBinThreads)
-            if (hist[t]) atomicAdd(&B.tile_count[t], hist[t]);
-}
-
-// One block: exclusive scan of the tile counts into entry offsets (the fill
-// cursors) and the item list (runs of at most `item_entries` entries per tile).
-__global__ void __launch_bounds__(kScanThreads) k_bin_scan(OneView vs, uint32_t item_entries) {
-    __shared__ uint32_t wsum[2][kScanThreads / 64];
-    __shared__ uint32_t carry[2];
-    const lh_view& v = vs.v;
-    const Bins B = bins(v);
     const uint32_t tiles = B.L.tiles, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (threadIdx.x == 0) carry[0] = carry[1] = 0;
-    __syncthreads();
-    for (uint32_t t0 = 0; t0 < tiles; t0 += kScanThreads) {
-        const uint32_t t = t0 + threadIdx.x;
-        const uint32_t c = t < tiles ? B.tile_count[t] : 0u;
-        const uint32_t ni = (c + item_entries - 1) / item_entries;
-        const uint32_t ic = wave_inclusive_scan(c), ii = wave_inclusive_scan(ni);
+    const bool wide = tiles > kHistTiles;
+    uint32_t *off = shared, *item_off = shared + kHistTiles, *cnt = shared + kHistTiles;
+    auto items_of = [&](uint32_t c) { return (c + item_entries - 1) / item_entries; };
+    auto put_item = [&](uint32_t t, uint32_t at, uint32_t c, uint32_t item, uint32_t j) {
+        if (item + j >= B.L.item_capacity) return;
+        const uint32_t b = at + j * item_entries, e = min(b + item_entries, at + c);
+        B.items[item + j] = TileItem{t, b, e | (c <= item_entries ? lhs::kItemOnly : 0u)};
+    };
+    {
+        const uint32_t per = (tiles + kBinThreads - 1) / kBinThreads, t0 = threadIdx.x * per, t1 = min(t0 + per, tiles);
+        uint32_t n = 0, ni = 0;
+        for (uint32_t t = t0; t < t1; t++) {
+            const uint32_t c = B.tile_count[tile_word(t, tiles)];
+            n += c;
+            ni += items_of(c);
+        }
+        const uint32_t in = wave_scan_add(n), ii = wave_scan_add(ni);
         if (lane == 63) {
-            wsum[0][wave] = ic;
+            wsum[0][wave] = in;
             wsum[1][wave] = ii;
         }
         __syncthreads();
-        uint32_t bc = carry[0], bi = carry[1];
+        uint32_t at = in - n, item = ii - ni;
         for (uint32_t w = 0; w < wave; w++) {
-            bc += wsum[0][w];
-            bi += wsum[1][w];
+            at += wsum[0][w];
+            item += wsum[1][w];
         }
-        const uint32_t off = bc + ic - c, ioff = bi + ii - ni;
-        if (t < tiles) {
-            B.tile_cursor[t] = off;
-            for (uint32_t j = 0; j < ni; j++) {
-                const uint32_t it = ioff + j;
-                if (it < B.L.item_capacity) {
-                    const uint32_t b = off + j * item_entries, e = min(b + item_entries, off + c);
-                    B.items[it] = TileItem{t, b, e | (ni == 1 ? lhs::kItemOnly : 0u)};
-                }
+        for (uint32_t t = t0; t < t1; t++) {
+            const uint32_t c = B.tile_count[tile_word(t, tiles)];
+            off[t] = at;
+            if (!wide)
+                item_off[t] = item;
+            else if (blockIdx.x == 0)
+                for (uint32_t j = 0; j < items_of(c); j++) put_item(t, at, c, item, j);
+            at += c;
+            item += items_of(c);
+        }
+        if (blockIdx.x == 0 && threadIdx.x == kBinThreads - 1) {
+            v.counters[LH_CNT_TILE_ITEMS] = min(item, B.L.item_capacity);
+            v.counters[LH_CNT_TILE_NEXT] = 0;  // the tile raster's work queue starts empty
+        }
+        __syncthreads();
+        if (!wide)
+            for (uint32_t t = blockIdx.x * (kBinThreads / 64) + wave; t < tiles; t += gridDim.x * (kBinThreads / 64)) {
+                const uint32_t c = B.tile_count[tile_word(t, tiles)];
+                for (uint32_t j = lane; j < items_of(c); j += 64) put_item(t, off[t], c, item_off[t], j);
             }
-        }
-        __syncthreads();
-        if (threadIdx.x == kScanThreads - 1) {
-            carry[0] = off + c;
-            carry[1] = ioff + ni;
-        }
-        __syncthreads();
+        __syncthreads();  // item_off becomes cnt
     }
-    if (threadIdx.x == 0) {
-        v.counters[LH_CNT_TILE_ITEMS] = min(carry[1], B.L.item_capacity);
-        v.counters[LH_CNT_TILE_NEXT] = 0;  // the tile raster's work queue starts empty
-    }
-}
-
-// One thread per binned draw: its entries at the tiles' cursors.  Per run of
-// kBinChunk draws a block counts its entries per tile in LDS, reserves each
-// tile's range with one device atomic, then hands out the slots in LDS.
-__global__ void __launch_bounds__(kBinThreads) k_bin_fill(OneView vs, PassSet ps) {
-    __shared__ uint32_t cnt[kHistTiles];
-    const lh_view& v = vs.v;
-    const Segments<OneView> seg(vs, ps);
-    const uint32_t nb = binned_draws(seg, v);
-    const Bins B = bins(v);
     auto binned = [&](uint32_t g, uint32_t& rect, uint32_t& parts) {
         if (g >= nb) return false;
         const BinHeader h = B.hdr[g];
@@ -347,39 +314,31 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_fill(OneView vs, PassSet ps
         parts = 1u << lhs::parts_log2(h.ntri);
         return h.ntri != 0 && (h.ntri & lhs::kBinDirect) == 0;
     };
-    if (B.L.tiles > kHistTiles) {
+    auto put = [&](uint32_t at, uint32_t g, uint32_t parts) {
+        for (uint32_t q = 0; q < parts; q++)
+            if (at + q < B.L.entry_capacity) B.entries[at + q] = g | (q << lhs::kEntryPartShift);
+    };
+    if (wide) {
         for (uint32_t g = blockIdx.x * kBinThreads + threadIdx.x; g < nb; g += gridDim.x * kBinThreads) {
             uint32_t rect, parts;
             if (binned(g, rect, parts))
-                for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) {
-                    const uint32_t at = atomicAdd(&B.tile_cursor[t], parts);
-                    for (uint32_t q = 0; q < parts; q++)
-                        if (at + q < B.L.entry_capacity) B.entries[at + q] = g | (q << lhs::kEntryPartShift);
-                });
+                for_each_tile(rect, B.L.tiles_x,
+                              [&](uint32_t t) { put(off[t] + atomicAdd(&B.tile_cursor[tile_word(t, tiles)], parts), g, parts); });
         }
         return;
     }
-    for (uint32_t c0 = blockIdx.x * kBinChunk; c0 < nb; c0 += gridDim.x * kBinChunk) {
-        for (uint32_t t = threadIdx.x; t < B.L.tiles; t += kBinThreads) cnt[t] = 0;
+    for (uint32_t c0 = blockIdx.x * kBinThreads; c0 < nb; c0 += gridDim.x * kBinThreads) {
+        for (uint32_t t = threadIdx.x; t < tiles; t += kBinThreads) cnt[t] = 0;
         __syncthreads();
-        for (uint32_t g = c0 + threadIdx.x; g < min(c0 + kBinChunk, nb); g += kBinThreads) {
-            uint32_t rect, parts;
-            if (binned(g, rect, parts))
-                for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) { atomicAdd(&cnt[t], parts); });
-        }
+        uint32_t rect = 0, parts = 0;
+        const uint32_t g = c0 + threadIdx.x;
+        const bool mine = binned(g, rect, parts);
+        if (mine) for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) { atomicAdd(&cnt[t], parts); });
         __syncthreads();
-        for (uint32_t t = threadIdx.x; t < B.L.tiles; t += kBinThreads)
-            if (cnt[t]) cnt[t] = atomicAdd(&B.tile_cursor[t], cnt[t]);
+        for (uint32_t t = threadIdx.x; t < tiles; t += kBinThreads)
+            if (cnt[t]) cnt[t] = off[t] + atomicAdd(&B.tile_cursor[tile_word(t, tiles)], cnt[t]);
         __syncthreads();
-        for (uint32_t g = c0 + threadIdx.x; g < min(c0 + kBinChunk, nb); g += kBinThreads) {
-            uint32_t rect, parts;
-            if (binned(g, rect, parts))
-                for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) {
-                    const uint32_t at = atomicAdd(&cnt[t], parts);
-                    for (uint32_t q = 0; q < parts; q++)
-                        if (at + q < B.L.entry_capacity) B.entries[at + q] = g | (q << lhs::kEntryPartShift);
-                });
-        }
+        if (mine) for_each_tile(rect, B.L.tiles_x, [&](uint32_t t) { put(atomicAdd(&cnt[t], parts), g, parts); });
         __syncthreads();
     }
 }
@@ -674,27 +633,28 @@ namespace lhk {
 
 template <bool ST>
 hipError_t raster_tiles(const lh_scene& s, const OneView& vs, const PassSet& ps, const RasterTuning& t,
-                        hipStream_t st) {
+                        bool bins_clear, hipStream_t st) {
     const uint32_t item_entries = std::min(std::max(t.tile_item_entries, lhs::kMinItemEntries), 64u * kTileWaves);
+    if (!bins_clear) {
+        mark("bin_reset_view", st);
+        hipLaunchKernelGGL(k_bin_reset, dim3(8), dim3(256), 0, st, vs);
+    }
     mark("bin_meshlets_view", st);
-    hipLaunchKernelGGL(k_bin_meshlets<0>, dim3(t.meshlet_blocks), dim3(64), 0, st, s, vs, ps);
-    // the draw count is on the device: grids sized for the view's draw capacity
-    const uint32_t chunks = std::max<uint32_t>(1, (std::min(vs.v.draw_capacity, 1u << 22) + kBinChunk - 1) / kBinChunk);
-    const uint32_t bin_blocks = std::min<uint32_t>(chunks, 256);
-    mark("bin_count_view", st);
-    hipLaunchKernelGGL(k_bin_count, dim3(bin_blocks), dim3(kBinThreads), 0, st, vs, ps);
-    mark("bin_scan_view", st);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kScanThreads), 0, st, vs, item_entries);
+    const uint32_t blocks = std::min<uint32_t>(kBinBlocks, std::max(s.total_meshlets, 1u));
+    hipLaunchKernelGGL(k_bin_meshlets<0>, dim3(blocks), dim3(64), 0, st, s, vs, ps);
+    // the draw count is on the device: the grid is sized for the most draws
+    const uint32_t most = std::min(std::min(vs.v.draw_capacity, vs.v.bin_capacity), std::max(s.total_meshlets, 1u));
+    const uint32_t chunks = std::max<uint32_t>(1, (std::min(most, 1u << 22) + kBinThreads - 1) / kBinThreads);
     mark("bin_fill_view", st);
-    hipLaunchKernelGGL(k_bin_fill, dim3(bin_blocks), dim3(kBinThreads), 0, st, vs, ps);
+    hipLaunchKernelGGL(k_bin_fill, dim3(std::min<uint32_t>(chunks, 256)), dim3(kBinThreads), 0, st, vs, ps, item_entries);
     mark("tile_raster_view", st);
     hipLaunchKernelGGL((k_tile_raster<ST>), dim3(t.tile_blocks), dim3(kTileThreads), 0, st, vs, ps);
     return hipGetLastError();
 }
 
-template hipError_t raster_tiles<false>(const lh_scene&, const OneView&, const PassSet&, const RasterTuning&,
+template hipError_t raster_tiles<false>(const lh_scene&, const OneView&, const PassSet&, const RasterTuning&, bool,
                                         hipStream_t);
-template hipError_t raster_tiles<true>(const lh_scene&, const OneView&, const PassSet&, const RasterTuning&,
+template hipError_t raster_tiles<true>(const lh_scene&, const OneView&, const PassSet&, const RasterTuning&, bool,
                                        hipStream_t);
 
 }  // namespace lhk

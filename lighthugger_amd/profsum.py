@@ -26,9 +26,8 @@ from pathlib import Path
 FRAME_KERNELS = {
     "tile_raster_view": "k_tile_raster<false>",
     "bin_meshlets_view": "k_bin_meshlets<0>",
-    "bin_count_view": "k_bin_count",
-    "bin_scan_view": "k_bin_scan",
     "bin_fill_view": "k_bin_fill",
+    "bin_reset_view": "k_bin_reset",
     # with the tiled raster on, the per-meshlet kernel of the main view runs as
     # raster_direct_view (the draws the bins left); otherwise as raster_meshlets_view
     "raster_direct_view": "k_raster_meshlets<0, lhd::OneView, false>",
