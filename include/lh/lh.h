@@ -65,6 +65,8 @@ typedef void* lh_stream; /* hipStream_t */
                                   bin_capacity, or a screen rectangle over LH_TILE_MAX_RECT tiles) */
 #define LH_CNT_BACKWARD_TICKET 60 /* lh_resolve_backward: blocks done; zero between calls (the view reset
                                      zeroes it, the call's last block sets it back to zero) */
+#define LH_CNT_DEPTH_TICKET 61 /* lh_frame of a small scene: blocks done of the depth reduction; zero
+                                  between calls */
 #define LH_NUM_COUNTERS 64
 #define LH_OVERFLOW_INSTANCES 0x1u
 #define LH_OVERFLOW_DRAWS 0x2u

@@ -43,13 +43,22 @@ hipError_t record_frame(const lh_scene& s, const lh_view& v, hipStream_t st) {
     // The attachment clears (src/rendering.cpp:206-211, :384) ride on the
     // meshlet culls: the view's cull clears the visibility buffer (and the
     // tiled raster's counts), the cascades' cull the shadow maps, each before the raster that writes them.
-    hipError_t e = view_reset(vs, st);
-    if (e == hipSuccess) e = cull_instances(s, vs, false, st);
+    hipError_t e;
+    if (s.num_instances <= kSmallReset) {
+        e = reset_cull_instances(s, vs, st);
+    } else {
+        e = view_reset(vs, st);
+        if (e == hipSuccess) e = cull_instances(s, vs, false, st);
+    }
     const uint32_t bins = v.bin_capacity > 0 ? kClearBins : 0u;
     if (e == hipSuccess) e = cull_meshlets(s, vs, 0, 1, tuning_for(v).cull_blocks, st, kClearVisbuffer | bins);
     if (e == hipSuccess) e = raster_main(s, vs, tuning_for(v), st, bins != 0);
-    if (e == hipSuccess) e = depth_bounds(vs, px, st);
-    if (e == hipSuccess) e = fit_cull_instances_shadow(s, vs, st);
+    if (s.num_instances <= kSmallFit) {
+        if (e == hipSuccess) e = depth_fit_cull(s, vs, st);
+    } else {
+        if (e == hipSuccess) e = depth_bounds(vs, px, st);
+        if (e == hipSuccess) e = fit_cull_instances_shadow(s, vs, st);
+    }
     if (e == hipSuccess) e = cull_meshlets(s, vs, 1, LH_NUM_CASCADES, tuning_for(v).cull_blocks, st, kClearShadowMaps);
     if (e == hipSuccess) e = raster(s, vs, 1, LH_NUM_CASCADES, tuning_for(v).raster, st);
     if (e == hipSuccess) e = resolve(s, vs, 0, lh_resolve_params{}, st);

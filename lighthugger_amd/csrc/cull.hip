@@ -5,6 +5,8 @@
 //   k_cull_instances          cull_instances     src/shaders/cull_instances.comp:7-27
 //                             cull_instances_shadows               :31-56
 //   k_fit_cull_instances_shadow  generate_shadow_matrices + cull_instances_shadows
+//   k_reset_cull_instances    the first and third in one block (small scenes)
+//   k_depth_fit_cull          read_depth + the fifth (small scenes)
 //   k_cull_meshlets           write_draw_calls(_shadows)  src/shaders/write_draw_calls.comp:7-117
 //
 // The prefix-sum append keeps the reference's single 64-bit atomic per append
@@ -17,6 +19,7 @@
 // Every kernel is templated on its view source (one view, or a table of views
 // indexed by blockIdx.z) so a batch of views runs the same arithmetic.
 #include "cascade.h"
+#include "depth.h"
 #include "hiz.h"
 #include "kernels.h"
 #include "lh_device.h"
@@ -234,6 +237,109 @@ __global__ void __launch_bounds__(256) k_fit_cull_instances_shadow(lh_scene s, V
     wave_prefix_append(v, 1 + c, visible, i, value);
 }
 
+// ---- small scenes ----
+// A frame of a small scene is a chain of launches of which each costs about
+// 4.6 us whatever it does, so two pairs of dependent launches are one for
+// scenes that a block can cull by itself in that time.
+
+// The view reset and the main view's instance cull of a scene of at most
+// kSmallReset instances, one per thread of one block: the append is a block
+// scan.  (For more the two launches are as fast: 2,000 instances took one
+// block 14 us against 14.)
+__global__ void __launch_bounds__(lhk::kSmallReset) k_reset_cull_instances(lh_scene s, OneView vs) {
+    constexpr uint32_t kWaves = lhk::kSmallReset / 64;
+    __shared__ uint32_t sums[kWaves], counts[kWaves];
+    const lh_view& v = vs.v;
+    const Uniforms& u = *v.uniforms;
+    const uint32_t i = threadIdx.x, wave = i >> 6;
+    bool visible = false;
+    uint32_t value = 0;
+    if (i < min(u.num_instances, s.num_instances)) {
+        const Instance& in = s.instances[i];
+        const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
+        visible = !cull_sphere(in, mi.bounding_sphere, u);
+        value = visible ? mi.num_meshlets : 0u;
+    }
+    const uint64_t m = ballot(visible);
+    uint32_t sum = wave_scan_add(value), slot = lanes_below(m);
+    if (lane_id() == 63) {
+        sums[wave] = sum;
+        counts[wave] = uint32_t(__popcll(m));
+    }
+    __syncthreads();
+    uint32_t total = 0, count = 0;
+    for (uint32_t w = 0; w < kWaves; w++) {
+        if (w < wave) sum += sums[w], slot += counts[w];
+        total += sums[w], count += counts[w];
+    }
+    uint64_t* sec = sector(v, 0);
+    if (visible && slot < v.instance_capacity)
+        reinterpret_cast<PrefixSumValue*>(sec + 1)[slot] = PrefixSumValue{i, sum};
+    if (i < LH_NUM_COUNTERS) v.counters[i] = i == LH_CNT_OVERFLOW && count > v.instance_capacity ? LH_OVERFLOW_INSTANCES : 0u;
+    if (i < LH_NUM_PASSES) sector(v, i)[0] = i == 0 ? uint64_t(total) | (uint64_t(count) << 32) : 0ull;
+    if (i == 0) {
+        v.misc->min_depth = 0xFFFFFFFFu;
+        v.misc->max_depth = 0u;
+    }
+}
+
+// The depth bounds, the cascade fit and the shadow instance cull of a scene of
+// at most kSmallFit instances: the last block of the depth pass to finish (a
+// ticket in the view's counters) fits the cascades and culls, one cascade per
+// wave, so each wave appends to a sector of its own without atomics.
+__global__ void __launch_bounds__(256) k_depth_fit_cull(lh_scene s, OneView vs) {
+    __shared__ uint32_t smin[4], smax[4], last;
+    __shared__ LhMat4 views[LH_NUM_CASCADES];
+    __shared__ float radii[LH_NUM_CASCADES];
+    const lh_view& v = vs.v;
+    depth::block_bounds(v, smin, smax);
+    if (threadIdx.x == 0) {
+        __threadfence();  // this block's bounds before its ticket
+        last = atomicAdd(&v.counters[LH_CNT_DEPTH_TICKET], 1u) == gridDim.x - 1 ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();  // every ticket before the bounds are read
+    const Uniforms& u = *v.uniforms;
+    const uint32_t min_bits = __hip_atomic_load(&v.misc->min_depth, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t max_bits = __hip_atomic_load(&v.misc->max_depth, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < LH_NUM_CASCADES) {
+        const cascade::Fit f = cascade::fit(u, min_bits, max_bits, threadIdx.x);
+        views[threadIdx.x] = f.view;
+        radii[threadIdx.x] = f.radius;
+        cascade::store(*v.misc, threadIdx.x, f);
+    }
+    if (threadIdx.x == 0) {
+        v.counters[LH_CNT_DEPTH_TICKET] = 0;
+        if (min_bits == 0xFFFFFFFFu) atomicOr(&v.counters[LH_CNT_FLAGS], LH_FLAG_EMPTY_VIEW);
+    }
+    __syncthreads();
+    const uint32_t n = min(u.num_instances, s.num_instances), c = threadIdx.x >> 6;
+    uint64_t* sec = sector(v, 1 + c);
+    PrefixSumValue* vals = reinterpret_cast<PrefixSumValue*>(sec + 1);
+    uint32_t sum = 0, count = 0;
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane_id();
+        bool visible = false;
+        uint32_t value = 0;
+        if (i < n) {
+            const Instance& in = s.instances[i];
+            const MeshInfo& mi = mesh_info_at(in.mesh_info_address);
+            visible = !cull_sphere_shadow(in, mi.bounding_sphere, views, radii, c);
+            value = visible ? mi.num_meshlets : 0u;
+        }
+        const uint64_t m = ballot(visible);
+        const uint32_t incl = wave_scan_add(value), slot = count + lanes_below(m);
+        if (visible && slot < v.instance_capacity) vals[slot] = PrefixSumValue{i, sum + incl};
+        sum += uint32_t(__builtin_amdgcn_readlane(int(incl), 63));
+        count += uint32_t(__popcll(m));
+    }
+    if (lane_id() == 0) {
+        sec[0] = uint64_t(sum) | (uint64_t(count) << 32);
+        if (count > v.instance_capacity) atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_INSTANCES);
+    }
+}
+
 // One pass per blockIdx.y (pass = pass0 + blockIdx.y), one view per
 // blockIdx.z; grid-stride over the meshlets of the pass's visible instances.
 // With LH_VIEW_HIZ (single view) the main-view survivors are split: large or
@@ -335,6 +441,21 @@ template <class VS>
 hipError_t view_reset(const VS& vs, hipStream_t st) {
     mark("view_reset", st);
     hipLaunchKernelGGL(k_view_reset<VS>, dim3(1, 1, vs.count()), dim3(64), 0, st, vs);
+    return hipGetLastError();
+}
+
+hipError_t reset_cull_instances(const lh_scene& s, const lhd::OneView& vs, hipStream_t st) {
+    // the profile keeps the passes' names: the launch counts for the last one
+    mark("view_reset", st);
+    mark("cull_instances", st);
+    hipLaunchKernelGGL(k_reset_cull_instances, dim3(1), dim3(kSmallReset), 0, st, s, vs);
+    return hipGetLastError();
+}
+
+hipError_t depth_fit_cull(const lh_scene& s, const lhd::OneView& vs, hipStream_t st) {
+    mark("depth_bounds", st);
+    mark("fit_cull_instances_shadow", st);
+    hipLaunchKernelGGL(k_depth_fit_cull, dim3(depth::blocks(uint64_t(vs.v.width) * vs.v.height)), dim3(256), 0, st, s, vs);
     return hipGetLastError();
 }
 

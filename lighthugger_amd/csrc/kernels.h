@@ -57,6 +57,11 @@ template <class VS>
 hipError_t clear_targets(const VS& vs, uint64_t max_pixels, hipStream_t st);
 template <class VS>
 hipError_t cull_instances(const lh_scene& s, const VS& vs, bool shadow, hipStream_t st);
+// Small scenes: view reset + main-view instance cull in one block, and depth
+// bounds + cascade fit + shadow instance cull in one launch.
+constexpr uint32_t kSmallReset = 1024, kSmallFit = 256;  // instances
+hipError_t reset_cull_instances(const lh_scene& s, const lhd::OneView& vs, hipStream_t st);
+hipError_t depth_fit_cull(const lh_scene& s, const lhd::OneView& vs, hipStream_t st);
 // generate_shadow_matrices + cull_instances_shadows in one launch.
 template <class VS>
 hipError_t fit_cull_instances_shadow(const lh_scene& s, const VS& vs, hipStream_t st);
