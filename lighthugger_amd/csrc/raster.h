@@ -603,6 +603,22 @@ LH_DEV void wave_spread(int32_t* own, uint32_t lane, uint32_t n, F&& f) {
     }
 }
 
+// Part `part` of 2^lg equal parts of a triangle: rows (or runs of pixels) dealt
+// out one by one.
+struct Share {
+    uint32_t part = 0, lg = 0;
+    LH_DEV uint32_t count(uint32_t rows) const { return (rows + ((1u << lg) - 1u) - part) >> lg; }
+    LH_DEV uint32_t nth(uint32_t k) const { return (k << lg) + part; }
+    LH_DEV int32_t first(uint32_t k, uint32_t run) const { return int32_t(k + part * run); }
+};
+// log2 of the waves that share each of n triangles: while that leaves a wave of
+// `waves` no more than `each` of them.
+LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t most) {
+    uint32_t lg = 0;
+    while (lg < most && (n << (lg + 1)) <= waves * each && waves >> (lg + 1)) lg++;
+    return lg;
+}
+
 // Rasterizes entries [from, from + n) of the queue, n <= 64, one per lane.
 // Boxes of up to kLanePx pixels (most of a dense scene's) are walked by their
 // own lane.  The others are spread over the wave twice: first their rows, one
@@ -616,7 +632,7 @@ LH_DEV void wave_spread(int32_t* own, uint32_t lane, uint32_t n, F&& f) {
 constexpr int32_t kLanePx = 4;
 template <int KIND, bool ST, bool ALPHA, bool EARLY, class Q, class A>
 LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q, A& alpha, uint32_t from, uint32_t n,
-                         uint32_t lane, Tally<ST>& tally) {
+                         uint32_t lane, Tally<ST>& tally, Share share = {}) {
     lds_order();
     uint32_t rows = 0;
     float inv_area = 0.0f;
@@ -624,7 +640,7 @@ LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q
         const QueuedTri t = load_tri(q, from + lane, p.W, p.H);
         inv_area = rcp_exact(float(t.area()));
         if constexpr (ALPHA) alpha.store(lane, shading::alpha_setup(s, M, t.id));
-        if (!ALPHA && __mul24(t.w, t.h) <= kLanePx) {
+        if (!ALPHA && share.lg == 0 && __mul24(t.w, t.h) <= kLanePx) {
             for (int32_t y = 0; y < t.h; y++) {
                 RowEdges r(t, y);
                 for (int32_t x = 0; x < t.w; x++) {
@@ -635,10 +651,11 @@ LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q
                 }
             }
         } else {
-            rows = uint32_t(t.h);
+            rows = share.count(uint32_t(t.h));
         }
     }
-    wave_spread(q.own, lane, rows, [&](int32_t o, uint32_t y, bool active) {
+    wave_spread(q.own, lane, rows, [&](int32_t o, uint32_t k, bool active) {
+        const uint32_t y = share.nth(k);
         uint32_t columns = 0, row = 0;  // row: first column | y << 8 | triangle << 16
         if (active) {
             const QueuedTri t = load_tri(q, from + uint32_t(o), p.W, p.H);

@@ -222,6 +222,7 @@ LH_DEV uint32_t clip_polygon(f4& v, uint32_t n, uint32_t lane, float4* poly) {
 // Triangles over kNarrow whose pixel box holds at most this many pixels are
 // rasterized by one wave alone; larger ones by the whole block.
 constexpr int32_t kWaveBoxPx = 4096;
+constexpr uint32_t kMaxShareLog2 = 3;
 
 // float(e), rounded once, for |e| < 2^53: exact as a double first (four
 // instructions; the direct conversion takes a dozen).
@@ -285,9 +286,10 @@ LH_DEV void raster_box(const lh_scene& s, const lh_view& v, const Pass& p, const
 // queue: triangles just over the medium extent) go through raster_queue
 // together, pass by pass; a wider one is rasterized by its wave alone when its
 // box holds at most kWaveBoxPx pixels, and by the block's four waves together
-// above.  Clip-crossing triangles: a block takes one at a time; its waves all
-// clip it (they need no exchange to agree) and share the pieces of the fan:
-// a narrow piece goes to one wave, a wide one to the whole block.
+// above.  Clip-crossing triangles: a block takes one at a time (several blocks
+// a part each where there are few); its waves all clip it (they need no
+// exchange to agree) and share the pieces of the fan: a narrow piece goes to
+// one wave, a wide one to the whole block.
 //
 // ALPHA selects the entries of alpha-clip geometry (alpha test per sample), so
 // the opaque instantiation keeps its small register footprint; the alpha one
@@ -321,16 +323,13 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
     auto& alpha = alphas4[wave];
     const Queues qs = queues(v);
     Tally<ST> tally;
-    auto raster_narrow = [&](uint32_t n, const Pass& p) {
+    auto raster_narrow = [&](uint32_t n, const Pass& p, Share share) {
         LhMat4 M{};
         if constexpr (ALPHA) M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
-        raster_queue<KIND, ST, ALPHA, !ST>(s, M, p, queue, alpha, 0, n, lane, tally);
+        raster_queue<KIND, ST, ALPHA, !ST>(s, M, p, queue, alpha, 0, n, lane, tally, share);
         lds_order();
         tally.flush(v, p.pass);
     };
-    // Entry of lane l of wave w in the round that starts at b0.  Neighbours in
-    // the queue are neighbours on a mesh and of much the same size, so a
-    // wave's entries lie `waves` apart: a run of large ones is shared out.
     const uint32_t waves = gridDim.x * 4;
     // The draws that the tiled raster left because of their size (few): their
     // triangles within the medium extent; the others are queued already.
@@ -363,16 +362,30 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
                 const uint64_t pm = ballot(push);
                 if (pm == 0) continue;
                 if (push) queue.store(lanes_below(pm), wv, ts, (h.mid << LH_KEY_TRI_BITS) | t);
-                raster_narrow(uint32_t(__popcll(pm)), p);
+                raster_narrow(uint32_t(__popcll(pm)), p, Share{});
             }
         }
     }
-    auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + blockIdx.x * 4 + w + l * waves; };
+    // Entry of lane l of wave w in the round that starts at b0.  Neighbours in
+    // the queue are neighbours on a mesh and of much the same size, so a
+    // wave's entries lie apart: a run of large ones is shared out.
+    // Where a wave would hold few entries, up to 2^kMaxShareLog2 waves take a
+    // part of each instead (their lanes have room for all those entries at
+    // once): the last wave to end is the one with the largest triangles, 200 us
+    // after the rest when one alone walked 4,096 pixels with an alpha test on
+    // each.  Alpha-clipped 1280x720, 33 k to 50 k entries, 197 of them wide:
+    // alpha launches 466 + 356 -> 146 + 151 us, the opaque one 56 -> 30; without
+    // wide ones 121 + 118 -> 96 + 133.  A limit of 8 or 32 entries a wave
+    // in place of 16 measures the same within the noise on opaque fields.
+    const uint32_t lg = share_out(count, waves, ALPHA ? 32 : 16, kMaxShareLog2);
+    const uint32_t groups = waves >> lg;
+    auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + ((blockIdx.x * 4 + w) >> lg) + l * groups; };
+    auto share = [&](uint32_t w) { return Share{(blockIdx.x * 4 + w) & ((1u << lg) - 1u), lg}; };
     uint32_t round = 0;
-    for (uint32_t b0 = 0; b0 + blockIdx.x * 4 < count; b0 += 64 * waves, round ^= 1) {  // block-uniform
+    for (uint32_t b0 = 0; b0 + (blockIdx.x * 4 >> lg) < count; b0 += 64 * groups, round ^= 1) {  // block-uniform
         const uint32_t e = entry(b0, wave, lane);
         BigTri b{};
-        const bool mine = e < count;
+        const bool mine = e < count && (blockIdx.x * 4 + wave) >> lg < groups;
         if (mine) b = qs.big[e];
         const int32_t xlo = b.xlo & 0x1FFF, ylo = b.ylo & ~kBigAlpha;
         const uint32_t pi = uint32_t(b.xlo) >> 13;
@@ -388,12 +401,12 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
             if (now)
                 queue.store(lanes_below(m), xlo, ylo, SV{b.X[0], b.Y[0], b.z[0]}, SV{b.X[1], b.Y[1], b.z[1]},
                             SV{b.X[2], b.Y[2], b.z[2]}, b.id);
-            raster_narrow(uint32_t(__popcll(m)), make_pass(v, ps.pass0 + q));
+            raster_narrow(uint32_t(__popcll(m)), make_pass(v, ps.pass0 + q), share(wave));
         }
         for (uint64_t m = ballot(wide && !huge); m; m &= m - 1) {
             const BigTri t = qs.big[entry(b0, wave, first_lane(m))];
             const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
-            raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, int32_t(lane), 64, tally);
+            raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, share(wave).first(lane, 64), 64 << lg, tally);
             tally.flush(v, p.pass);
         }
         const uint64_t hm = ballot(huge);
@@ -403,12 +416,14 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
             for (uint64_t m = giant[round][w]; m; m &= m - 1) {
                 const BigTri t = qs.big[entry(b0, w, first_lane(m))];
                 const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
-                raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, int32_t(threadIdx.x), 256, tally);
+                raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, share(w).first(threadIdx.x, 256), 256 << lg, tally);
                 tally.flush(v, p.pass);
             }
     }
-    for (uint32_t c = blockIdx.x; c < clips; c += gridDim.x) {
-        const uint2 e = qs.clip[c];
+    const uint32_t clip_lg = share_out(clips, gridDim.x, 1, kMaxShareLog2);
+    for (uint32_t c = blockIdx.x; c < clips << clip_lg; c += gridDim.x) {
+        const uint2 e = qs.clip[c >> clip_lg];
+        const Share part{c & ((1u << clip_lg) - 1u), clip_lg};
         if (((e.y & kClipAlpha) != 0) != ALPHA) continue;
         const uint32_t d = e.x >> LH_KEY_TRI_BITS, t = e.x & ((1u << LH_KEY_TRI_BITS) - 1), pi = e.y & ~kClipAlpha;
         const Pass p = make_pass(v, ps.pass0 + pi);
@@ -441,7 +456,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
         const uint64_t nm = ballot(narrow);
         if (nm) {
             if (narrow) queue.store(lanes_below(nm), xlo, ylo, v0, v1, v2, id);
-            raster_narrow(uint32_t(__popcll(nm)), p);
+            raster_narrow(uint32_t(__popcll(nm)), p, part);
         }
         for (uint64_t m = ballot(wide); m; m &= m - 1) {
             const uint32_t l = first_lane(m);
@@ -452,7 +467,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
             b.id = id;
             b.xlo = uint16_t(readlane(xlo, l)), b.ylo = uint16_t(readlane(ylo, l));
             b.xhi = uint16_t(readlane(xhi, l)), b.yhi = uint16_t(readlane(yhi, l));
-            raster_box<KIND, ST, ALPHA>(s, v, p, b, alpha, int32_t(threadIdx.x), 256, tally);
+            raster_box<KIND, ST, ALPHA>(s, v, p, b, alpha, part.first(threadIdx.x, 256), 256 << clip_lg, tally);
             tally.flush(v, p.pass);
         }
     }
