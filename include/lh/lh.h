@@ -328,8 +328,8 @@ lh_status lh_view_status(const lh_view* view, uint32_t* host_counters, lh_stream
  * reference, whose raster is fixed-function).  Results are independent of
  * them; the autotuner picks them per resolution class.  Process-global. */
 typedef struct lh_tuning {
-    uint32_t small_extent_px;  /* tiled main-view raster: boxes of at most this many pixels a side
-                                  (1..32) are rasterized by one lane */
+    uint32_t small_extent_px;  /* lower bound of medium_extent_px (1..32); boxes of a few pixels are
+                                  rasterized by one lane, by a limit of the kernels */
     uint32_t meshlet_blocks;   /* persistent grid of the per-meshlet raster (one wave per block) */
     uint32_t big_blocks;       /* persistent grid of the large-triangle raster */
     uint32_t clip_blocks;      /* no effect (must be non-zero): clip-crossing triangles run on the
@@ -343,8 +343,8 @@ typedef struct lh_tuning {
                                    is non-zero); 0: the per-meshlet raster.  The tiled raster wins when
                                    meshlets cover many pixels each; with a few pixels per meshlet (small
                                    views of dense scenes) the per-meshlet raster is cheaper. */
-    uint32_t shadow_small_extent_px;  /* the cascades' small_extent_px (0..32; 0 = small_extent_px): the
-                                         shadow maps' triangles and raster differ from the main view's */
+    uint32_t shadow_small_extent_px;  /* lower bound of the cascades' medium_extent_px (0..32; 0 =
+                                         small_extent_px) */
     uint32_t shadow_medium_extent_px; /* the cascades' medium_extent_px (0..64; 0 = medium_extent_px) */
 } lh_tuning;
 /* lh_set_tuning sets every class at once, lh_get_tuning reads class 1;

@@ -22,15 +22,13 @@ from . import abi
 TUNING_FILE = Path(__file__).resolve().parent / "tuning.json"
 
 SPACE = {
-    "small_extent_px": [2, 3, 4, 6, 8],
-    "medium_extent_px": [8, 12, 16, 32, 64],
-    "meshlet_blocks": [4096, 8192, 16384],
-    "big_blocks": [512, 2048],
+    "medium_extent_px": [8, 12, 16, 24, 32],
+    "meshlet_blocks": [8192, 16384, 24576, 32768, 49152],
+    "big_blocks": [1024, 2048, 4096],
     "cull_blocks": [512, 1024, 2048],
-    "tile_item_entries": [32, 64, 128],
+    "tile_item_entries": [32, 48, 64, 128],
     "tile_blocks": [768, 1024, 2048],
     "tile_raster": [0, 1],
-    "shadow_small_extent_px": [0, 4, 6, 8],
     "shadow_medium_extent_px": [0, 8, 16, 32],
 }
 FIELDS = ("small_extent_px", "meshlet_blocks", "big_blocks", "clip_blocks", "cull_blocks", "medium_extent_px",

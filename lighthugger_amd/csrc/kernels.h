@@ -14,7 +14,7 @@ namespace lhk {
 
 // Raster tunables (chosen by the autotuner; output is independent of them).
 struct RasterTuning {
-    uint32_t small_extent_px = 4;   // in-lane raster when the vertex bbox is within this many pixels
+    uint32_t small_extent_px = 4;   // kept as set: the least medium extent
     uint32_t medium_extent_px = 64; // wave-cooperative raster up to this extent
     uint32_t meshlet_blocks = 8192; // persistent grid of the per-meshlet kernel (64-thread blocks)
     uint32_t big_blocks = 2048;     // persistent grid of the large-triangle kernel (256-thread blocks)
@@ -22,7 +22,7 @@ struct RasterTuning {
     uint32_t tile_item_entries = 64; // tiled main-view raster: binned meshlets per work item (>= 8)
     uint32_t tile_blocks = 1024;    // tiled main-view raster: persistent grid (512-thread blocks)
     uint32_t tile_raster = 1;       // main view through the tiled raster (when bin_capacity > 0)
-    uint32_t shadow_small_extent_px = 0;  // the cascades' small_extent_px (0: the same)
+    uint32_t shadow_small_extent_px = 0;  // the cascades' least medium extent (0: the same)
     uint32_t shadow_medium_extent_px = 0; // the cascades' medium_extent_px (0: the same)
 };
 

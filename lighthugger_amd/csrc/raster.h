@@ -35,6 +35,7 @@ struct SV {
 
 // One render target of a launch.
 struct Pass {
+    static constexpr int32_t kLanePx = 4;  // boxes up to this many pixels are walked by one lane
     uint32_t pass, W, H;
     uint64_t* vis;
     uint32_t* depth;
@@ -46,7 +47,6 @@ struct Pass {
 // LH_CNT_CLIP / LH_CNT_BIG + pass0.
 struct PassSet {
     uint32_t pass0, n;
-    int32_t small_extent;   // subpixels: the tiled raster's in-lane boxes, up to this side
     int32_t medium_extent;  // subpixels: larger triangles go to the large-triangle queue (<= 64 px)
     uint32_t phase2;        // main view, second occlusion phase: draws from LH_CNT_HIZ_PHASE1 on
     uint32_t direct;        // single view: rasterize the draws the tiled raster left on its direct list
@@ -470,11 +470,11 @@ LH_DEV void queue_big(const lh_view& v, uint32_t pass0, bool pred, const WaveVer
 // snapped vertices relative to the origin's pixel corner (16 bits each), the three depths and the key's id; triangles are
 // oriented to positive area.  A round adds at most 64 entries to at most 63.
 constexpr uint32_t kQueue = 128;
-template <uint32_t N>
+template <uint32_t N, class Own = int32_t>
 struct TriQueueOf {
     uint4 box[N];     // xlo | ylo << 16, v0, v1, v2 (x & 0xFFFF | y << 16)
     uint4 att[N];     // z0, z1, z2, id
-    int32_t own[64];  // owners of a pass's runs
+    Own own[64];      // owners of a pass's runs
     // a triangle of positive area; (xlo, ylo): first pixel of its clamped box
     LH_DEV void store(uint32_t k, int32_t xlo, int32_t ylo, const SV& v0, const SV& v1, const SV& v2, uint32_t id) {
         auto rel = [&](const SV& v) {
@@ -571,13 +571,18 @@ LH_DEV void clip_row(int32_t e, int32_t s, int32_t m, int32_t& lo, int32_t& hi) 
         hi = -1;
 }
 
-// Depth test of the pixel at (x, y) of a queued triangle's box.
-template <int KIND, bool ST, bool EARLY, class F>
-LH_DEV void raster_pixel(const Pass& p, const QueuedTri& t, float inv_area, int32_t e1, int32_t e2, int32_t x, int32_t y,
+// Depth test of the pixel at (x, y) of a queued triangle's box: in the pass's
+// render target, or in another one that has its own test (a tile in LDS).
+template <int KIND, bool ST, bool EARLY, class P, class F>
+LH_DEV void raster_pixel(const P& p, const QueuedTri& t, float inv_area, int32_t e1, int32_t e2, int32_t x, int32_t y,
                          Tally<ST>& tally, F&& visible) {
     const int32_t px = t.xlo + x, py = t.ylo + y;
     const float l1 = float(e1) * inv_area, l2 = float(e2) * inv_area;
-    fragment<KIND, ST, EARLY>(p, px, py, (t.z0 + l1 * t.d10) + l2 * t.d20, t.id, tally, [&] { return visible(px, py); });
+    const float z = (t.z0 + l1 * t.d10) + l2 * t.d20;
+    if constexpr (std::is_same<P, Pass>::value)
+        fragment<KIND, ST, EARLY>(p, px, py, z, t.id, tally, [&] { return visible(px, py); });
+    else
+        tally.hit(p.put(px, py, z, t.id));
 }
 
 // Numbers the `n` pieces of work of each lane in lane order and hands them out
@@ -585,17 +590,17 @@ LH_DEV void raster_pixel(const Pass& p, const QueuedTri& t, float inv_area, int3
 // (the owners' registers are read across lanes).  A lane finds the owner of
 // its piece as the last lane whose first piece is at or before it: first
 // pieces are marked in LDS, and a running maximum spreads the marks.
-template <class F>
-LH_DEV void wave_spread(int32_t* own, uint32_t lane, uint32_t n, F&& f) {
+template <class Own, class F>
+LH_DEV void wave_spread(Own* own, uint32_t lane, uint32_t n, F&& f) {
     const uint32_t incl = wave_scan_add(n), excl = incl - n;
     const uint32_t total = readlane_u32(incl, 63);
     int32_t carry = 0;
     for (uint32_t base = 0; base < total; base += 64) {
         own[lane] = -1;
         lds_order();
-        if (n && excl - base < 64u) own[excl - base] = int32_t(lane);  // excl >= base, unsigned
+        if (n && excl - base < 64u) own[excl - base] = Own(lane);  // excl >= base, unsigned
         lds_order();
-        const int32_t o = max(wave_scan_max(own[lane]), carry);
+        const int32_t o = max(wave_scan_max(int32_t(own[lane])), carry);
         lds_order();
         carry = __builtin_amdgcn_readlane(o, 63);
         const uint32_t k = base + lane;
@@ -620,7 +625,7 @@ LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t mo
 }
 
 // Rasterizes entries [from, from + n) of the queue, n <= 64, one per lane.
-// Boxes of up to kLanePx pixels (most of a dense scene's) are walked by their
+// Boxes of up to P::kLanePx pixels (most of a dense scene's) are walked by their
 // own lane.  The others are spread over the wave twice: first their rows, one
 // per lane, each cut to the columns that the triangle covers (exactly, so no
 // pixel is tested again); then the rows' covered pixels in runs of up to four.
@@ -629,9 +634,8 @@ LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t mo
 // dearer than the coverage: its runs are single pixels.  Against boxes walked
 // in runs of four with the edges tested at each pixel: the main views of 12
 // cameras 2.77 -> 1.96 ms, the alpha-clipped 720p view 1.12 -> 0.56 ms.
-constexpr int32_t kLanePx = 4;
-template <int KIND, bool ST, bool ALPHA, bool EARLY, class Q, class A>
-LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q, A& alpha, uint32_t from, uint32_t n,
+template <int KIND, bool ST, bool ALPHA, bool EARLY, class P, class Q, class A>
+LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const P& p, Q& q, A& alpha, uint32_t from, uint32_t n,
                          uint32_t lane, Tally<ST>& tally, Share share = {}) {
     lds_order();
     uint32_t rows = 0;
@@ -640,7 +644,7 @@ LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const Pass& p, Q& q
         const QueuedTri t = load_tri(q, from + lane, p.W, p.H);
         inv_area = rcp_exact(float(t.area()));
         if constexpr (ALPHA) alpha.store(lane, shading::alpha_setup(s, M, t.id));
-        if (!ALPHA && share.lg == 0 && __mul24(t.w, t.h) <= kLanePx) {
+        if (!ALPHA && share.lg == 0 && __mul24(t.w, t.h) <= P::kLanePx) {
             for (int32_t y = 0; y < t.h; y++) {
                 RowEdges r(t, y);
                 for (int32_t x = 0; x < t.w; x++) {

@@ -360,129 +360,36 @@ LH_DEV bool tile_fragment(uint64_t* tile, int32_t lx, int32_t ly, float z, uint3
     return true;
 }
 
-// Materializes v in a register at this point.  The triangle's values come
-// from LDS reads; left to itself the compiler recomputes them inside a pixel
-// loop, and the LDS-counter wait those reads need then also waits for every
-// depth atomic the loop has issued.
-template <class T>
-LH_DEV void pin(T& v) {
-    asm volatile("" : "+v"(v));
-}
-
-// Coverage of one pixel centre by an oriented triangle (exact integer edges).
-template <class E>
-LH_DEV bool inside(E e0, E e1, E e2, bool tl0, bool tl1, bool tl2) {
-    return (e0 > 0 || (e0 == 0 && tl0)) && (e1 > 0 || (e1 == 0 && tl1)) && (e2 > 0 || (e2 == 0 && tl2));
-}
-
-// In-lane raster of a triangle whose box inside the tile is small (at most
-// small_extent pixels a side): the lane walks the box itself.
-template <bool ST>
-LH_DEV void tile_lane(uint64_t* tile, int32_t ox, int32_t oy, SV a, SV b, SV c, int32_t xlo, int32_t xhi, int32_t ylo,
-                      int32_t yhi, float inv_area, uint32_t id, Tally<ST>& tally) {
-    pin(a.X), pin(a.Y), pin(b.X), pin(b.Y), pin(c.X), pin(c.Y);
-    float z0 = a.z, d10 = b.z - a.z, d20 = c.z - a.z;
-    pin(z0), pin(d10), pin(d20), pin(inv_area);
-    const bool tl0 = top_left(b.X, b.Y, c.X, c.Y), tl1 = top_left(c.X, c.Y, a.X, a.Y), tl2 = top_left(a.X, a.Y, b.X, b.Y);
-    for (int32_t py = ylo; py <= yhi; py++) {
-        const int32_t Py = py * 256 + 128;
-        for (int32_t px = xlo; px <= xhi; px++) {
-            const int32_t Px = px * 256 + 128;
-            const int32_t e0 = (c.X - b.X) * (Py - b.Y) - (c.Y - b.Y) * (Px - b.X);
-            const int32_t e1 = (a.X - c.X) * (Py - c.Y) - (a.Y - c.Y) * (Px - c.X);
-            const int32_t e2 = (b.X - a.X) * (Py - a.Y) - (b.Y - a.Y) * (Px - a.X);
-            if (inside(e0, e1, e2, tl0, tl1, tl2)) {
-                const float l1 = float(e1) * inv_area, l2 = float(e2) * inv_area;
-                tally.hit(tile_fragment(tile, px - ox, py - oy, (z0 + l1 * d10) + l2 * d20, id));
-            }
-        }
-    }
-}
-
-// Load-balanced raster of one round of triangles (one per lane) over the
-// wave.  A lane's clamped box is cut into runs of up to kRun pixels along its
-// rows (`n` runs, 0 for none); the runs are numbered in lane order (exclusive
-// scan) and handed out 64 at a time, so a wave spends ceil(sum n / 64) passes
-// on a round instead of the largest box.  A lane finds the triangle of its
-// run as the last one starting at or before it (start lanes mark their first
-// run in `own`, an inclusive max-scan spreads the marks), fetches the
-// triangle's corners, box and 1/area from that lane and its snapped vertices
-// from the wave's LDS copy, and steps the edge functions along the run.
-constexpr int32_t kRun = 4;
-LH_DEV int32_t runs_per_row(int32_t w) { return (w + kRun - 1) / kRun; }
-
-template <bool ST>
-LH_DEV void tile_expand(uint64_t* tile, int32_t ox, int32_t oy, int32_t* own, const int32_t* sX, const int32_t* sY,
-                        const float* sZ, uint32_t tri, uint32_t n, int32_t xlo, int32_t ylo, int32_t w, float inv_area,
-                        uint32_t mid, uint32_t lane, Tally<ST>& tally) {
-    const uint32_t incl = wave_scan_add(n), excl = incl - n;
-    const uint32_t total = uint32_t(__builtin_amdgcn_readlane(int(incl), 63));
-    const int32_t box = (xlo - ox) | ((ylo - oy) << 8) | (w << 16);  // tile-relative origin and width
-    int32_t carry = 0;
-    for (uint32_t base = 0; base < total; base += 64) {
-        own[lane] = -1;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (n && excl >= base && excl < base + 64) own[excl - base] = int32_t(lane);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        int32_t o = max(wave_scan_max(own[lane]), carry);
-        carry = __builtin_amdgcn_readlane(o, 63);
-        // every lane takes part in the fetches (the owner lanes are active)
-        const uint32_t otri = __shfl(tri, o, 64);
-        const int32_t obox = __shfl(box, o, 64);
-        const uint32_t oex = __shfl(excl, o, 64);
-        const float oinv = __shfl(inv_area, o, 64);
-        const uint32_t omid = uint32_t(__shfl(int(mid), o, 64));
-        const uint32_t k = base + lane;
-        if (k < total) {
-            // run (local % wr, local / wr) of the owner's box; local < 4096, wr <= 16
-            const int32_t ow = obox >> 16, wr = runs_per_row(ow);
-            const int32_t local = int32_t(k - oex);
-            int32_t q = int32_t(float(local) * __builtin_amdgcn_rcpf(float(wr)));
-            int32_t r = local - q * wr;
-            if (r < 0) q--, r += wr;
-            if (r >= wr) q++, r -= wr;
-            const int32_t lx0 = (obox & 255) + kRun * r, ly = ((obox >> 8) & 255) + q;
-            const int32_t len = min(kRun, ow - kRun * r);
-            const uint32_t i0 = otri & 255u, i1 = (otri >> 8) & 255u, i2 = (otri >> 16) & 255u;
-            const SV a{sX[i0], sY[i0], sZ[i0]}, b{sX[i1], sY[i1], sZ[i1]}, c{sX[i2], sY[i2], sZ[i2]};
-            const int32_t Px = (ox + lx0) * 256 + 128, Py = (oy + ly) * 256 + 128;
-            int32_t e0 = (c.X - b.X) * (Py - b.Y) - (c.Y - b.Y) * (Px - b.X);
-            int32_t e1 = (a.X - c.X) * (Py - c.Y) - (a.Y - c.Y) * (Px - c.X);
-            int32_t e2 = (b.X - a.X) * (Py - a.Y) - (b.Y - a.Y) * (Px - a.X);
-            int32_t s0 = -(c.Y - b.Y) * 256, s1 = -(a.Y - c.Y) * 256, s2 = -(b.Y - a.Y) * 256;
-            bool tl0 = top_left(b.X, b.Y, c.X, c.Y), tl1 = top_left(c.X, c.Y, a.X, a.Y),
-                 tl2 = top_left(a.X, a.Y, b.X, b.Y);
-            float z0 = a.z, d10 = b.z - a.z, d20 = c.z - a.z, inv = oinv;
-            pin(z0), pin(d10), pin(d20), pin(inv), pin(s0), pin(s1), pin(s2);
-            const uint32_t id = (omid << LH_KEY_TRI_BITS) | (otri >> 24);
-            for (int32_t j = 0; j < len; j++) {
-                if (inside(e0, e1, e2, tl0, tl1, tl2)) {
-                    const float l1 = float(e1) * inv, l2 = float(e2) * inv;
-                    tally.hit(tile_fragment(tile, lx0 + j, ly, (z0 + l1 * d10) + l2 * d20, id));
-                }
-                e0 += s0;
-                e1 += s1;
-                e2 += s2;
-            }
-        }
-    }
-}
+// The LDS tile as a render target of raster_queue; coordinates are the tile's.
+struct TileTarget {
+    uint64_t* tile;
+    uint32_t W, H;  // of the part inside the view
+    // An LDS depth test costs a lane less than a device atomic: 0, 4, 8, 12, 16,
+    // 24 px: stress tiles 503, 469, 457, 449, 443, 438 us, 1920x1080 84, 81,
+    // 78, 74, 72, 72, 1280x720 50, 50, 52, 51, 51, 55.
+    static constexpr int32_t kLanePx = 16;
+    LH_DEV bool put(int32_t x, int32_t y, float z, uint32_t id) const { return tile_fragment(tile, x, y, z, id); }
+};
 
 // Persistent blocks of kTileWaves waves over the work items.  Item: clear the
 // LDS tile; each wave takes every kTileWaves-th entry (one binned meshlet),
 // with the entry list of the item held one per lane and the next meshlet's
-// cache lines requested while the current one is rasterized.  When an entry
-// and the next hold at most 64 triangles together (an entry averages about
-// 35), both go through one round: the second's vertices at LDS slots
-// 64..127, its triangles on the lanes after the first's, each lane with its
-// own meshlet id.  Then the covered pixels go out: a plain store when the
-// item is the tile's only one (the visibility buffer holds the clear value
-// there, as nothing else has drawn yet), an atomicMin otherwise and in the
-// second occlusion phase.  Six waves per SIMD (80 VGPRs; the pairing's
-// registers would otherwise take the kernel to five).
+// cache lines requested while the current one is set up.  The triangles whose
+// box holds a pixel centre of the tile are collected in the wave's queue and
+// rasterized when it is full (raster.h).  Then the covered pixels go out: a
+// plain store when the item is the tile's only one (the visibility buffer holds
+// the clear value there, as nothing else has drawn yet), an atomicMin otherwise
+// and in the second occlusion phase.
+//
+// Bound by VALU issue.  With a round's triangles on one entry's lanes and boxes
+// walked in runs of four, 27 of 64 lanes were active: 1920x1080 101 us, 720p
+// 77, the 3840x2160 field 152, 20,000 instances 557; with the queue and the
+// exact row spans 72, 51, 124, 443.
+//
+// LDS is what limits the blocks of a compute unit to three (six waves per
+// SIMD): vertices are kept relative to the tile in 16 bits.  A triangle of at
+// most 64 px that touches the tile lies within them; the clamp keeps any other
+// vertex on its side of the tile.
 struct CacheLanes {
     int32_t X, Y;
     float Z;
@@ -505,19 +412,21 @@ LH_DEV CacheLanes load_cache(const BinCache& c, uint32_t lane, uint32_t first) {
 template <bool ST>
 __global__ void __launch_bounds__(kTileThreads) LH_WAVES_ATTR(6) k_tile_raster(OneView vs, PassSet ps) {
     __shared__ uint64_t tile[kTile * kTile];
-    __shared__ int32_t sX[kTileWaves][128], sY[kTileWaves][128];
-    __shared__ float sZ[kTileWaves][128];
-    __shared__ int32_t own[kTileWaves][64];
+    __shared__ uint2 verts8[kTileWaves][64];  // x & 0xFFFF | y << 16 (subpixels of the tile), z
+    __shared__ TriQueueOf<64, int8_t> queues8[kTileWaves];
     const lh_view& v = vs.v;
     const Bins B = bins(v);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t n_items = min(v.counters[LH_CNT_TILE_ITEMS], B.L.item_capacity);
     const int32_t W = int32_t(v.width), H = int32_t(v.height);
+    uint2* const verts = verts8[wave];
+    auto& queue = queues8[wave];
+    NoAlpha none;
     Tally<ST> tally;
     // Block b starts on item b; each further item comes from a queue, so a
     // block that drew light items takes more of them instead of idling while
-    // the heavy ones finish.
-    __shared__ uint32_t next_item;
+    // the heavy ones finish.  (The word is a vertex's between the barriers.)
+    uint32_t& next_item = verts8[0][0].x;
     for (uint32_t it = blockIdx.x; it < n_items;) {
         const TileItem item = B.items[it];
         const int32_t ox = int32_t(item.tile % B.L.tiles_x) * int32_t(kTile);
@@ -541,72 +450,47 @@ __global__ void __launch_bounds__(kTileThreads) LH_WAVES_ATTR(6) k_tile_raster(O
             cur = load_cache(B.cache[uint32_t(readlane(int32_t(my_g), 0))], lane,
                              uint32_t(readlane(int32_t(my_first), 0)));
         __syncthreads();
-        for (uint32_t k = 0; k < mine;) {
+        const TileTarget target{tile, uint32_t(ex - ox + 1), uint32_t(ey - oy + 1)};
+        uint32_t held = 0;  // triangles in the queue
+        auto flush = [&] {
+            if (held) raster_queue<0, ST, false, false>(lh_scene{}, LhMat4{}, target, queue, none, 0, held, lane, tally);
+            held = 0;
+            lds_order();
+        };
+        for (uint32_t k = 0; k < mine; k++) {
             const uint32_t ntri = uint32_t(readlane(int32_t(my_count), k)), mid = uint32_t(readlane(int32_t(my_mid), k));
-            const uint32_t ntri2 = k + 1 < mine ? uint32_t(readlane(int32_t(my_count), k + 1)) : 65u;
-            const bool pair = ntri + ntri2 <= 64u;  // wave-uniform
-            const uint32_t mid2 = pair ? uint32_t(readlane(int32_t(my_mid), k + 1)) : 0u;
-            CacheLanes next{};
+            auto rel = [](int32_t X, int32_t o) { return min(max(X - o * 256, -32768), 32767); };
+            lds_order();
+            verts[lane] = make_uint2((uint32_t(rel(cur.X, ox)) & 0xFFFFu) | uint32_t(rel(cur.Y, oy)) << 16,
+                                     __float_as_uint(cur.Z));
+            lds_order();
+            const uint32_t tris[2] = {cur.t0, cur.t1};
             if (k + 1 < mine)
-                next = load_cache(B.cache[uint32_t(readlane(int32_t(my_g), k + 1))], lane,
-                                  uint32_t(readlane(int32_t(my_first), k + 1)));
-            sX[wave][lane] = cur.X;
-            sY[wave][lane] = cur.Y;
-            sZ[wave][lane] = cur.Z;
-            uint32_t tri_pair = cur.t0, lane_mid = mid;
-            if (pair) {
-                sX[wave][64 + lane] = next.X;
-                sY[wave][64 + lane] = next.Y;
-                sZ[wave][64 + lane] = next.Z;
-                const uint32_t from = uint32_t(__shfl(int(next.t0), int((lane - ntri) & 63u), 64));
-                if (lane >= ntri) {
-                    tri_pair = from + 0x404040u;  // corners of the second entry at slots 64..127
-                    lane_mid = mid2;
-                }
-                // the second entry is consumed: its registers take the request
-                // of the entry after the pair
-                if (k + 2 < mine)
-                    next = load_cache(B.cache[uint32_t(readlane(int32_t(my_g), k + 2))], lane,
-                                      uint32_t(readlane(int32_t(my_first), k + 2)));
+                cur = load_cache(B.cache[uint32_t(readlane(int32_t(my_g), k + 1))], lane,
+                                 uint32_t(readlane(int32_t(my_first), k + 1)));
+#pragma unroll
+            for (uint32_t round = 0; round < 2; round++) {
+                if (round * 64 >= ntri) break;
+                const uint32_t tri = tris[round];
+                const uint2 a = verts[tri & 63u], b = verts[(tri >> 8) & 63u], c = verts[(tri >> 16) & 63u];
+                const int32_t ax = lo16(a.x), ay = hi16(a.x), bx = lo16(b.x), by = hi16(b.x), cx = lo16(c.x), cy = hi16(c.x);
+                const int32_t xlo = max((min(ax, min(bx, cx)) + 127) >> 8, 0);
+                const int32_t ylo = max((min(ay, min(by, cy)) + 127) >> 8, 0);
+                const int32_t xhi = min((max(ax, max(bx, cx)) - 128) >> 8, int32_t(target.W) - 1);
+                const int32_t yhi = min((max(ay, max(by, cy)) - 128) >> 8, int32_t(target.H) - 1);
+                const bool push = lane + 64 * round < ntri && xlo <= xhi && ylo <= yhi;
+                const uint64_t pm = ballot(push);
+                const uint32_t n = uint32_t(__popcll(pm));
+                if (n == 0) continue;
+                if (held + n > 64) flush();
+                if (push)
+                    queue.store(held + lanes_below(pm), xlo, ylo, SV{ax, ay, __uint_as_float(a.y)},
+                                SV{bx, by, __uint_as_float(b.y)}, SV{cx, cy, __uint_as_float(c.y)},
+                                (mid << LH_KEY_TRI_BITS) | (tri >> 24));
+                held += n;
             }
-            const uint32_t total = pair ? ntri + ntri2 : ntri;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            for (uint32_t round = 0; round < 2 && round * 64 < total; round++) {
-                const uint32_t tri = pair ? tri_pair : (round ? cur.t1 : cur.t0);
-                uint32_t n = 0;
-                int32_t xlo = 0, ylo = 0, w = 1;
-                float inv_area = 0.0f;
-                if (lane + 64 * round < total) {
-                    const uint32_t i0 = tri & 255u, i1 = (tri >> 8) & 255u, i2 = (tri >> 16) & 255u;
-                    const SV a{sX[wave][i0], sY[wave][i0], sZ[wave][i0]};
-                    const SV b{sX[wave][i1], sY[wave][i1], sZ[wave][i1]};
-                    const SV c{sX[wave][i2], sY[wave][i2], sZ[wave][i2]};
-                    const int32_t minX = min(a.X, min(b.X, c.X)), maxX = max(a.X, max(b.X, c.X));
-                    const int32_t minY = min(a.Y, min(b.Y, c.Y)), maxY = max(a.Y, max(b.Y, c.Y));
-                    xlo = max((minX + 127) >> 8, ox);
-                    const int32_t xhi = min((maxX - 128) >> 8, ex);
-                    ylo = max((minY + 127) >> 8, oy);
-                    const int32_t yhi = min((maxY - 128) >> 8, ey);
-                    if (xlo <= xhi && ylo <= yhi) {
-                        w = xhi - xlo + 1;
-                        const int32_t h = yhi - ylo + 1;
-                        // positive area (oriented by the binning), every value within int32 (<= 64 px)
-                        inv_area = rcp_exact(float((b.X - a.X) * (c.Y - a.Y) - (b.Y - a.Y) * (c.X - a.X)));
-                        if (max(w, h) * 256 <= ps.small_extent)
-                            tile_lane<ST>(tile, ox, oy, a, b, c, xlo, xhi, ylo, yhi, inv_area,
-                                          (lane_mid << LH_KEY_TRI_BITS) | (tri >> 24), tally);
-                        else
-                            n = uint32_t(runs_per_row(w) * h);
-                    }
-                }
-                tile_expand<ST>(tile, ox, oy, own[wave], sX[wave], sY[wave], sZ[wave], tri, n, xlo, ylo, w, inv_area,
-                                lane_mid, lane, tally);
-            }
-            k += pair ? 2u : 1u;
-            cur = next;
         }
+        flush();
         tally.flush(v, 0);
         __syncthreads();
         const bool only = (item.end & lhs::kItemOnly) && !ps.phase2;
