@@ -421,7 +421,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
                 tally.flush(v, p.pass);
             }
     }
-    const uint32_t clip_lg = share_out(clips, gridDim.x, 1, kMaxShareLog2);
+    const uint32_t clip_lg = share_out(clips, waves, 1, kMaxShareLog2);
     for (uint32_t c = blockIdx.x; c < clips << clip_lg; c += gridDim.x) {
         const uint2 e = qs.clip[c >> clip_lg];
         const Share part{c & ((1u << clip_lg) - 1u), clip_lg};
