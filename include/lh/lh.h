@@ -340,9 +340,11 @@ typedef struct lh_tuning {
     uint32_t tile_item_entries; /* tiled main-view raster: binned meshlets per work item (8..512; 0 = 64) */
     uint32_t tile_blocks;       /* tiled main-view raster: persistent grid of 512-thread blocks (0 = 1024) */
     uint32_t tile_raster;       /* 1: the main view goes through the tiled raster (when its bin_capacity
-                                   is non-zero); 0: the per-meshlet raster.  The tiled raster wins when
-                                   meshlets cover many pixels each; with a few pixels per meshlet (small
-                                   views of dense scenes) the per-meshlet raster is cheaper. */
+                                   is non-zero); 0: the per-meshlet raster.  The tiled raster wins where
+                                   a million meshlets lie over one another in a large view (20,000
+                                   instances seen whole, 5120x2880: 7.0 against 7.7 ms); below that
+                                   its binning costs more than it saves (a 2,000-instance field,
+                                   1920x1080: 433 against 390 us, 3840x2160: 967 against 931) */
     uint32_t shadow_small_extent_px;  /* lower bound of the cascades' medium_extent_px (0..32; 0 =
                                          small_extent_px) */
     uint32_t shadow_medium_extent_px; /* the cascades' medium_extent_px (0..64; 0 = medium_extent_px) */

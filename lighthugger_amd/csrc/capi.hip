@@ -50,7 +50,7 @@ hipError_t record_frame(const lh_scene& s, const lh_view& v, hipStream_t st) {
         e = view_reset(vs, st);
         if (e == hipSuccess) e = cull_instances(s, vs, false, st);
     }
-    const uint32_t bins = v.bin_capacity > 0 ? kClearBins : 0u;
+    const uint32_t bins = v.bin_capacity > 0 && tuning_for(v).raster.tile_raster ? kClearBins : 0u;
     if (e == hipSuccess) e = cull_meshlets(s, vs, 0, 1, tuning_for(v).cull_blocks, st, kClearVisbuffer | bins);
     if (e == hipSuccess) e = raster_main(s, vs, tuning_for(v), st, bins != 0);
     if (s.num_instances <= kSmallFit) {
