@@ -47,8 +47,10 @@ typedef void* lh_stream; /* hipStream_t */
 
 /* Device counters of one view (u32 each). */
 #define LH_CNT_DRAWS 0     /* + pass: surviving meshlets of the pass (may exceed draw_capacity) */
-#define LH_CNT_BIG 8       /* + pass: triangles queued for the large-triangle raster (the pieces of
-                              clipped triangles are rasterized without being queued) */
+#define LH_CNT_BIG 8       /* + pass: triangles for the large-triangle raster's queue (may exceed
+                              big_capacity: the per-meshlet raster draws the rest itself, or queues
+                              them for clipping; the pieces of clipped triangles are rasterized
+                              without being queued) */
 #define LH_CNT_CLIP 16     /* + pass: triangles queued for clipping */
 #define LH_CNT_OVERFLOW 24 /* bit mask of LH_OVERFLOW_* */
 #define LH_CNT_FLAGS 25    /* bit mask of LH_FLAG_* */
@@ -70,7 +72,7 @@ typedef void* lh_stream; /* hipStream_t */
 #define LH_NUM_COUNTERS 64
 #define LH_OVERFLOW_INSTANCES 0x1u
 #define LH_OVERFLOW_DRAWS 0x2u
-#define LH_OVERFLOW_BIG 0x4u
+#define LH_OVERFLOW_BIG 0x4u /* tiled raster: a large triangle found the queue full and is missing */
 #define LH_OVERFLOW_CLIP 0x8u
 #define LH_FLAG_EMPTY_VIEW 0x1u /* no geometry: depth bounds stayed at their reset values */
 

@@ -449,17 +449,19 @@ LH_DEV void queue_clip(const lh_view& v, uint32_t pass0, bool pred, uint32_t d, 
     else
         atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_CLIP);
 }
-LH_DEV void queue_big(const lh_view& v, uint32_t pass0, bool pred, const WaveVerts& wv, const TriSetup& ts, uint32_t id,
-                      uint32_t pi, bool alpha) {
-    if (ballot(pred) == 0) return;
-    const uint32_t slot = wave_append(&v.counters[LH_CNT_BIG + pass0], pred);
-    if (!pred) return;
+LH_DEV void store_big(BigTri* q, const WaveVerts& wv, const TriSetup& ts, uint32_t id, uint32_t pi, bool alpha) {
     const SV v0{ts.a.x, ts.a.y, wv.Z[ts.i0]}, v1{ts.b.x, ts.b.y, wv.Z[ts.i1]}, v2{ts.c.x, ts.c.y, wv.Z[ts.i2]};
-    if (slot < v.big_capacity)
-        store_big(queues(v).big + slot, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id, ts.xlo, ts.xhi, ts.ylo,
-                  ts.yhi, pi, alpha);
-    else
-        atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
+    store_big(q, v0, ts.swapped ? v2 : v1, ts.swapped ? v1 : v2, id, ts.xlo, ts.xhi, ts.ylo, ts.yhi, pi, alpha);
+}
+// Returns whether the lane's triangle found the queue full.
+LH_DEV bool queue_big(const lh_view& v, uint32_t pass0, bool pred, const WaveVerts& wv, const TriSetup& ts, uint32_t id,
+                      uint32_t pi, bool alpha) {
+    if (ballot(pred) == 0) return false;
+    const uint32_t slot = wave_append(&v.counters[LH_CNT_BIG + pass0], pred);
+    if (!pred) return false;
+    if (slot >= v.big_capacity) return true;
+    store_big(queues(v).big + slot, wv, ts, id, pi, alpha);
+    return false;
 }
 
 // Triangles of up to kNarrow that are ready to be rasterized, collected over a

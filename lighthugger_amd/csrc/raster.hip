@@ -144,10 +144,18 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
             for (uint32_t round = 0; round * 64 < ntri; round++) {
                 const uint32_t t = lane + 64 * round;
                 const TriSetup ts = triangle_setup<KIND>(wv, f.corners(cur, lane, round), t < ntri, clean, ALPHA, p.W, p.H);
-                if (!clean) queue_clip(v, ps.pass0, ts.clip && !queued, d, t, pi, ALPHA);
-                const bool big = ts.inside && ts.extent > ps.medium_extent, push = ts.inside && !big;
+                const bool big = ts.inside && ts.extent > ps.medium_extent;
                 const uint32_t id = (cur.mid << LH_KEY_TRI_BITS) | t;
-                queue_big(v, ps.pass0, big && !queued, wv, ts, id, pi, ALPHA);
+                bool push = ts.inside && !big;
+                if (!clean || ballot(big && !queued)) {
+                    // A full queue (how many are queued depends on the extents,
+                    // which may not cost a picture): the wave keeps the triangle,
+                    // or, a wide one, the clip queue takes it (nothing is cut off
+                    // then).
+                    const bool full = queue_big(v, ps.pass0, big && !queued, wv, ts, id, pi, ALPHA);
+                    queue_clip(v, ps.pass0, (ts.clip && !queued) || (full && ts.extent > kNarrow), d, t, pi, ALPHA);
+                    push = push || (full && ts.extent <= kNarrow);
+                }
                 const uint64_t pm = ballot(push);
                 if (pm == 0) continue;
                 if (push) queue.store(held + lanes_below(pm), wv, ts, id);

@@ -176,7 +176,8 @@ __global__ void __launch_bounds__(64) LH_WAVES_ATTR(LH_BIN_WAVES) k_bin_meshlets
                 if (!clean) queue_clip(v, ps.pass0, ts.clip, d, t, 0, false);
                 // triangles over the medium extent: spread over many blocks by the large-triangle raster
                 const bool big = ts.inside && ts.extent > ps.medium_extent, front = ts.inside && !big;
-                queue_big(v, ps.pass0, big, wv, ts, (cur.mid << LH_KEY_TRI_BITS) | t, 0, false);
+                if (queue_big(v, ps.pass0, big, wv, ts, (cur.mid << LH_KEY_TRI_BITS) | t, 0, false))
+                    atomicOr(&v.counters[LH_CNT_OVERFLOW], LH_OVERFLOW_BIG);
                 const uint64_t fm = ballot(front);
                 if (front) {
                     xlo_m = min(xlo_m, ts.xlo), ylo_m = min(ylo_m, ts.ylo);
