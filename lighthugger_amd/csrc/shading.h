@@ -550,7 +550,8 @@ LH_DEV AlphaTri alpha_setup(const lh_scene& s, const LhMat4& m, uint32_t id) {
         const f3 w = mat4_point(in.transform, load_position(mi, vi));
         clip[j] = mat4_mul_vec4(m, f4{w.x, w.y, w.z, 1.0f});
         if (!(clip[j].w > 0.0f)) t.texture = UNUSED_TEXTURE_INDEX;
-        const f2 q = load_uv(mi, vi);
+        // (a mesh without a texture need not have uvs)
+        const f2 q = t.texture != UNUSED_TEXTURE_INDEX ? load_uv(mi, vi) : f2{0.0f, 0.0f};
         t.uv[j] = {q.x * ts.x, q.y * ts.y};
     }
     t.bary = bary_setup(clip[0], clip[1], clip[2]);
