@@ -192,8 +192,17 @@ LH_DEV f4 clip_point(f4 a, f4 b, float da, float db) {
 // cards at 720p: 1.07, 0.88, 0.71, 0.68, 0.67 ms a frame at 16, 12, 8, 6, 4 px).
 constexpr int32_t kAlphaMediumPx = 6;
 
-// A triangle clipped by six planes has at most nine corners.
-constexpr uint32_t kPolyMax = 12;
+// Corners that the clipped polygon may have in LDS.  A convex one has at most
+// nine after six planes, but corners that lie on a plane to within rounding may
+// alternate about it (ten occur), and each change of side adds a corner: a
+// plane makes at most m + floor(m / 2) of m corners, from 3 at most 4, 6, 9,
+// 13, 19, 28.
+constexpr uint32_t poly_corners(uint32_t planes) {
+    const uint32_t m = planes == 0 ? 3 : poly_corners(planes - 1);
+    return planes == 0 ? m : m + m / 2;
+}
+constexpr uint32_t kPolyMax = poly_corners(6);
+static_assert(kPolyMax == 28 && kPolyMax <= 64, "one corner per lane");
 
 // Clips a polygon held one corner per lane (lanes 0..n-1) by the six planes
 // and returns its number of corners (0 when nothing is left).  Per plane every
