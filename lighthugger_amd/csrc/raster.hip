@@ -241,6 +241,7 @@ LH_DEV uint32_t clip_polygon(f4& v, uint32_t n, uint32_t lane, float4* poly) {
 // rasterized by one wave alone; larger ones by the whole block.
 constexpr int32_t kWaveBoxPx = 4096;
 constexpr uint32_t kMaxShareLog2 = 3;
+constexpr uint32_t kDirectShareLog2 = 4;
 
 // float(e), rounded once, for |e| < 2^53: exact as a double first (four
 // instructions; the direct conversion takes a dozen).
@@ -349,8 +350,14 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
         tally.flush(v, p.pass);
     };
     const uint32_t waves = gridDim.x * 4;
-    // The draws that the tiled raster left because of their size (few): their
-    // triangles within the medium extent; the others are queued already.
+    // The draws that the tiled raster left because of their size (few, over
+    // LH_TILE_MAX_RECT tiles each): their triangles within the medium extent;
+    // the others are queued already.  A wave alone on one of them ends long
+    // after the rest, so up to 2^kDirectShareLog2 waves set up the same draw and
+    // take a part of its triangles' rows each.  Medium extent 64, frame of the
+    // field at 1920x1080 and 3840x2160: 882 and 1,746 us with one wave a draw,
+    // 539 and 1,109 with 4, 483 and 998 with 8, 448 and 959 with 16, 440 and 948
+    // with 32 (839 and 1,743 when a launch of its own drew them).
     if constexpr (KIND == 0 && !ALPHA && std::is_same<VS, OneView>::value) {
         __shared__ WaveVerts verts4[4];
         WaveVerts& wv = verts4[wave];
@@ -359,9 +366,11 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
         const uint32_t n = ps.direct ? min(v.counters[LH_CNT_TILE_DIRECT], L.direct_capacity) : 0u;
         const Segments<VS> seg(vs, ps);
         const Pass p = make_pass(v, ps.pass0);
-        for (uint32_t i = blockIdx.x * 4 + wave; i < n; i += waves) {
+        uint32_t lg = 0;
+        while (lg < kDirectShareLog2 && n << (lg + 1) <= waves) lg++;
+        for (uint32_t i = blockIdx.x * 4 + wave; i < n << lg; i += waves) {
             uint32_t view, pi, d;
-            seg.find(uniform_u32(list[i]) & ~lhs::kBinDirect, view, pi, d);
+            seg.find(uniform_u32(list[i >> lg]) & ~lhs::kBinDirect, view, pi, d);
             const DrawHead h = head_of_lane(load_head(s, p.draws[d]), 0);
             MeshletFetch f;
             f.request(h, lane);
@@ -380,7 +389,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
                 const uint64_t pm = ballot(push);
                 if (pm == 0) continue;
                 if (push) queue.store(lanes_below(pm), wv, ts, (h.mid << LH_KEY_TRI_BITS) | t);
-                raster_narrow(uint32_t(__popcll(pm)), p, Share{});
+                raster_narrow(uint32_t(__popcll(pm)), p, Share{i & ((1u << lg) - 1u), lg});
             }
         }
     }
