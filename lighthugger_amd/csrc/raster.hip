@@ -406,13 +406,24 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
     // in place of 16 measures the same within the noise on opaque fields.
     const uint32_t lg = share_out(count, waves, ALPHA ? 32 : 16, kMaxShareLog2);
     const uint32_t groups = waves >> lg;
-    auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + ((blockIdx.x * 4 + w) >> lg) + l * groups; };
-    auto share = [&](uint32_t w) { return Share{(blockIdx.x * 4 + w) & ((1u << lg) - 1u), lg}; };
+    // Number of the block's wave w.  A block's four waves follow one another,
+    // but in a queue with at most an entry for every other block each goes to a
+    // block of its own: four triangles over kWaveBoxPx in one block, one after the
+    // other and their samples behind a read of the target, outlast all else.
+    // 1,500 opaque triangles at 1920x1080, frame: of 150 px 325 -> 254 us (307
+    // in a form without the read), of 300 px 556 -> 323, of 20 px 123 -> 124;
+    // 4,000 of 60 px, over the limit, 244 (261 apart).  Alpha-clipped ones lose
+    // more by it (4,000 of 60 px 433 -> 644: neighbours share texels) than they
+    // gain.
+    const bool apart = !ALPHA && count << lg <= gridDim.x / 2;
+    auto number = [&](uint32_t w) { return apart ? blockIdx.x + w * gridDim.x : blockIdx.x * 4 + w; };
+    auto entry = [&](uint32_t b0, uint32_t w, uint32_t l) { return b0 + (number(w) >> lg) + l * groups; };
+    auto share = [&](uint32_t w) { return Share{number(w) & ((1u << lg) - 1u), lg}; };
     uint32_t round = 0;
-    for (uint32_t b0 = 0; b0 + (blockIdx.x * 4 >> lg) < count; b0 += 64 * groups, round ^= 1) {  // block-uniform
+    for (uint32_t b0 = 0; b0 + (number(0) >> lg) < count; b0 += 64 * groups, round ^= 1) {  // block-uniform
         const uint32_t e = entry(b0, wave, lane);
         BigTri b{};
-        const bool mine = e < count && (blockIdx.x * 4 + wave) >> lg < groups;
+        const bool mine = e < count && number(wave) >> lg < groups;
         if (mine) b = qs.big[e];
         const int32_t xlo = b.xlo & 0x1FFF, ylo = b.ylo & ~kBigAlpha;
         const uint32_t pi = uint32_t(b.xlo) >> 13;
