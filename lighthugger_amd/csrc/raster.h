@@ -170,6 +170,7 @@ template <bool ON>
 struct Tally {
     LH_DEV void hit(bool) {}
     LH_DEV void flush(const lh_view&, uint32_t) {}
+    LH_DEV void move_to(Tally*, uint32_t) {}
 };
 template <>
 struct Tally<true> {
@@ -185,6 +186,13 @@ struct Tally<true> {
             atomicAdd(&v.counters[LH_CNT_FRAGMENTS + pass], f);
             atomicAdd(&v.counters[LH_CNT_ATOMICS + pass], a);
         }
+        frags = atomics = 0;
+    }
+    // Adds the lane's counts to those of pass `pi` of sum[LH_NUM_CASCADES].
+    LH_DEV void move_to(Tally* sum, uint32_t pi) {
+#pragma unroll
+        for (uint32_t q = 0; q < LH_NUM_CASCADES; q++)
+            if (q == pi) sum[q].frags += frags, sum[q].atomics += atomics;
         frags = atomics = 0;
     }
 };

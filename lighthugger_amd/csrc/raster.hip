@@ -341,13 +341,20 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
     __shared__ std::conditional_t<ALPHA, AlphaStore, NoAlpha> alphas4[4];
     auto& alpha = alphas4[wave];
     const Queues qs = queues(v);
-    Tally<ST> tally;
+    // Statistics: each lane counts per pass of the set, and the block adds its
+    // counts to the view's once at the end: one pair of same-address atomics a
+    // block and pass, where a pair after every batch of triangles took this
+    // launch of the 1920x1080 field from 72 to 393 us.  (A form that flushed
+    // after every triangle, one to a block, once wrote wrong depths in frames with
+    // statistics; the cause was never found, so nothing is flushed between
+    // triangles.)
+    Tally<ST> tally, sums[LH_NUM_CASCADES];
     auto raster_narrow = [&](uint32_t n, const Pass& p, Share share) {
         LhMat4 M{};
         if constexpr (ALPHA) M = load_mat4(reinterpret_cast<uint64_t>(&view_matrix<KIND>(v, p.pass)));
         raster_queue<KIND, ST, ALPHA, !ST>(s, M, p, queue, alpha, 0, n, lane, tally, share);
         lds_order();
-        tally.flush(v, p.pass);
+        tally.move_to(sums, p.pass - ps.pass0);
     };
     const uint32_t waves = gridDim.x * 4;
     // The draws that the tiled raster left because of their size (few, over
@@ -445,7 +452,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
             const BigTri t = qs.big[entry(b0, wave, first_lane(m))];
             const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
             raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, share(wave).first(lane, 64), 64 << lg, tally);
-            tally.flush(v, p.pass);
+            tally.move_to(sums, p.pass - ps.pass0);
         }
         const uint64_t hm = ballot(huge);
         if (lane == 0) giant[round][wave] = hm;
@@ -455,7 +462,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
                 const BigTri t = qs.big[entry(b0, w, first_lane(m))];
                 const Pass p = make_pass(v, ps.pass0 + (uint32_t(t.xlo) >> 13));
                 raster_box<KIND, ST, ALPHA>(s, v, p, t, alpha, share(w).first(threadIdx.x, 256), 256 << lg, tally);
-                tally.flush(v, p.pass);
+                tally.move_to(sums, p.pass - ps.pass0);
             }
     }
     const uint32_t clip_lg = share_out(clips, waves, 1, kMaxShareLog2);
@@ -506,7 +513,22 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
             b.xlo = uint16_t(readlane(xlo, l)), b.ylo = uint16_t(readlane(ylo, l));
             b.xhi = uint16_t(readlane(xhi, l)), b.yhi = uint16_t(readlane(yhi, l));
             raster_box<KIND, ST, ALPHA>(s, v, p, b, alpha, part.first(threadIdx.x, 256), 256 << clip_lg, tally);
-            tally.flush(v, p.pass);
+            tally.move_to(sums, p.pass - ps.pass0);
+        }
+    }
+    if constexpr (ST) {
+        __shared__ uint32_t counts[4][2 * LH_NUM_CASCADES];
+#pragma unroll
+        for (uint32_t q = 0; q < LH_NUM_CASCADES; q++) {
+            const uint32_t f = wave_sum_u32(sums[q].frags), a = wave_sum_u32(sums[q].atomics);
+            if (lane == 0) counts[wave][2 * q] = f, counts[wave][2 * q + 1] = a;
+        }
+        __syncthreads();
+        const uint32_t q = threadIdx.x >> 1;
+        if (q < ps.n) {
+            uint32_t n = 0;
+            for (uint32_t w = 0; w < 4; w++) n += counts[w][threadIdx.x];
+            if (n) atomicAdd(&v.counters[(threadIdx.x & 1 ? LH_CNT_ATOMICS : LH_CNT_FRAGMENTS) + ps.pass0 + q], n);
         }
     }
 }
