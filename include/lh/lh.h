@@ -73,7 +73,9 @@ typedef void* lh_stream; /* hipStream_t */
 #define LH_OVERFLOW_INSTANCES 0x1u
 #define LH_OVERFLOW_DRAWS 0x2u
 #define LH_OVERFLOW_BIG 0x4u /* tiled raster: a large triangle found the queue full and is missing */
-#define LH_OVERFLOW_CLIP 0x8u
+#define LH_OVERFLOW_CLIP 0x8u /* a triangle found the clip queue full and is missing: a clip-crossing one, or
+                                 (per-meshlet raster) one over 120 px that had found the large-triangle
+                                 queue full, so that big_capacity is too small as well */
 #define LH_FLAG_EMPTY_VIEW 0x1u /* no geometry: depth bounds stayed at their reset values */
 
 /* lh_view.flags */

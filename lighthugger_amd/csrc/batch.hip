@@ -27,6 +27,7 @@ struct lh_batch {
     uint32_t* d_tiles = nullptr;
     uint32_t total_tiles = 0;
     uint64_t max_pixels = 0, max_shadow = 0;
+    bool short_queue = false;
     hipStream_t capture_stream = nullptr;
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -43,17 +44,20 @@ hipError_t record_batched(const lh_batch& b, hipStream_t st) {
     using namespace lhk;
     const lhd::ViewTable vt = table(b);
     const lh_scene& s = b.scene;
+    const Tuning& t = g_tunings[kBatchTuningClass];
+    RasterTuning rt = t.raster;
+    rt.short_queue = b.short_queue;
     hipError_t e = view_reset(vt, st);
     if (e == hipSuccess) e = clear_targets(vt, std::max(b.max_pixels, b.max_shadow), st);
     if (e == hipSuccess) e = cull_instances(s, vt, false, st);
-    if (e == hipSuccess) e = cull_meshlets(s, vt, 0, 1, g_tunings[kBatchTuningClass].cull_blocks, st);
+    if (e == hipSuccess) e = cull_meshlets(s, vt, 0, 1, t.cull_blocks, st);
     if (e == hipSuccess) e = plan_segments(vt, 0, 1, st);
-    if (e == hipSuccess) e = raster(s, vt, 0, 1, g_tunings[kBatchTuningClass].raster, st);
+    if (e == hipSuccess) e = raster(s, vt, 0, 1, rt, st);
     if (e == hipSuccess) e = depth_bounds(vt, b.max_pixels, st);
     if (e == hipSuccess) e = fit_cull_instances_shadow(s, vt, st);
-    if (e == hipSuccess) e = cull_meshlets(s, vt, 1, LH_NUM_CASCADES, g_tunings[kBatchTuningClass].cull_blocks, st);
+    if (e == hipSuccess) e = cull_meshlets(s, vt, 1, LH_NUM_CASCADES, t.cull_blocks, st);
     if (e == hipSuccess) e = plan_segments(vt, 1, LH_NUM_CASCADES, st);
-    if (e == hipSuccess) e = raster(s, vt, 1, LH_NUM_CASCADES, g_tunings[kBatchTuningClass].raster, st);
+    if (e == hipSuccess) e = raster(s, vt, 1, LH_NUM_CASCADES, rt, st);
     if (e == hipSuccess) e = resolve(s, vt, b.total_tiles, lh_resolve_params{}, st);
     return e;
 }
@@ -103,6 +107,7 @@ lh_status lh_batch_create(const lh_scene* scene, const lh_view* views, uint32_t 
         tiles[i + 1] = tiles[i] + ((v.width + 7) / 8) * ((v.height + 7) / 8);
         b->max_pixels = std::max<uint64_t>(b->max_pixels, uint64_t(v.width) * v.height);
         b->max_shadow = std::max<uint64_t>(b->max_shadow, uint64_t(v.shadow_size) * v.shadow_size);
+        b->short_queue = b->short_queue || v.big_capacity < lhk::kAmpleQueue;
     }
     b->total_tiles = tiles[n_views];
     const size_t seg_n = size_t(LH_NUM_CASCADES) * n_views + 1;

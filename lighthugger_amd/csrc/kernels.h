@@ -24,7 +24,13 @@ struct RasterTuning {
     uint32_t tile_raster = 1;       // main view through the tiled raster (when bin_capacity > 0)
     uint32_t shadow_small_extent_px = 0;  // the cascades' least medium extent (0: the same)
     uint32_t shadow_medium_extent_px = 0; // the cascades' medium_extent_px (0: the same)
+    bool short_queue = false;       // a batch view's big_capacity is below kAmpleQueue
 };
+
+// Large-triangle queues from this many entries on (the least of the Python
+// defaults) have room for every triangle over a low medium extent; a shorter
+// one was sized by its owner, for the extents of raster()'s short_queue.
+constexpr uint32_t kAmpleQueue = 1u << 18;
 
 struct Tuning {
     RasterTuning raster;

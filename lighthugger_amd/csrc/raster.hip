@@ -148,10 +148,8 @@ LH_DEV void raster_meshlets(const lh_scene& s, const VS& vs, const PassSet& ps) 
                 const uint32_t id = (cur.mid << LH_KEY_TRI_BITS) | t;
                 bool push = ts.inside && !big;
                 if (!clean || ballot(big && !queued)) {
-                    // A full queue (how many are queued depends on the extents,
-                    // which may not cost a picture): the wave keeps the triangle,
-                    // or, a wide one, the clip queue takes it (nothing is cut off
-                    // then).
+                    // A full queue: the wave keeps the triangle, or, a wide one, the
+                    // clip queue takes it (nothing is cut off then).
                     const bool full = queue_big(v, ps.pass0, big && !queued, wv, ts, id, pi, ALPHA);
                     queue_clip(v, ps.pass0, (ts.clip && !queued) || (full && ts.extent > kNarrow), d, t, pi, ALPHA);
                     push = push || (full && ts.extent <= kNarrow);
@@ -190,7 +188,7 @@ LH_DEV f4 clip_point(f4 a, f4 b, float da, float db) {
 // which spreads them over the chip: their samples are far dearer than opaque
 // ones, and a wave would keep its meshlet's to itself (1,500 alpha-clipped
 // cards at 720p: 1.07, 0.88, 0.71, 0.68, 0.67 ms a frame at 16, 12, 8, 6, 4 px).
-constexpr int32_t kAlphaMediumPx = 6;
+constexpr uint32_t kAlphaMediumPx = 6;
 
 // Corners that the clipped polygon may have in LDS.  A convex one has at most
 // nine after six planes, but corners that lie on a plane to within rounding may
@@ -566,7 +564,7 @@ namespace lhk {
 // covers only the draws it left.
 template <int KIND, bool ST, class VS>
 hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const RasterTuning& t, uint32_t big_blocks,
-                          bool bins_clear, hipStream_t st) {
+                          int32_t alpha_extent, bool bins_clear, hipStream_t st) {
     const uint32_t nv = vs.count();
     bool tiled = false;
     if constexpr (std::is_same<VS, OneView>::value)
@@ -596,7 +594,7 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
     if (alpha) {
         mark(KIND == 0 ? "raster_alpha_view" : "raster_alpha_shadow", st);
         PassSet pa = ps;
-        pa.medium_extent = std::min(ps.medium_extent, kAlphaMediumPx * 256);
+        pa.medium_extent = alpha_extent;
         hipLaunchKernelGGL((k_raster_alpha<KIND, VS, ST>), dim3(blocks), dim3(64), 0, st, s, vs, pa);
     }
     ps.direct = direct ? 1u : 0u;
@@ -612,14 +610,14 @@ hipError_t launch_kernels(const lh_scene& s, const VS& vs, PassSet ps, const Ras
 // Statistics are a single-view feature (LH_VIEW_STATISTICS).
 template <int KIND>
 hipError_t launch_set(const lh_scene& s, const OneView& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
-                      bool bins_clear, hipStream_t st) {
-    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, bb, bins_clear, st);
-    return launch_kernels<KIND, false>(s, vs, ps, t, bb, bins_clear, st);
+                      int32_t alpha_extent, bool bins_clear, hipStream_t st) {
+    if (vs.v.flags & LH_VIEW_STATISTICS) return launch_kernels<KIND, true>(s, vs, ps, t, bb, alpha_extent, bins_clear, st);
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, alpha_extent, bins_clear, st);
 }
 template <int KIND>
 hipError_t launch_set(const lh_scene& s, const ViewTable& vs, const PassSet& ps, const RasterTuning& t, uint32_t bb,
-                      bool bins_clear, hipStream_t st) {
-    return launch_kernels<KIND, false>(s, vs, ps, t, bb, bins_clear, st);
+                      int32_t alpha_extent, bool bins_clear, hipStream_t st) {
+    return launch_kernels<KIND, false>(s, vs, ps, t, bb, alpha_extent, bins_clear, st);
 }
 
 template <class VS>
@@ -633,13 +631,22 @@ hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npas
     const uint32_t small_sel = cascades && t.shadow_small_extent_px ? t.shadow_small_extent_px : t.small_extent_px;
     const uint32_t medium_sel = cascades && t.shadow_medium_extent_px ? t.shadow_medium_extent_px : t.medium_extent_px;
     const uint32_t small_px = std::min<uint32_t>(std::max<uint32_t>(small_sel, 1), 32);
-    const uint32_t medium_px = std::min<uint32_t>(std::max(medium_sel, small_px), 64);
+    // A low extent queues many times the triangles (12 px in place of 16 at
+    // 1920x1080: 80 k for 33 k), and a wide one that finds the queue full needs a
+    // place in the clip queue.  A short queue keeps the extents at which its
+    // owner found it long enough: 16 px, 64 px in a batch, alpha-clipped ones the
+    // same.
+    bool short_queue = t.short_queue;
+    if constexpr (std::is_same<VS, OneView>::value) short_queue = vs.v.big_capacity < kAmpleQueue;
+    const uint32_t least_px = !short_queue ? 1u : std::is_same<VS, OneView>::value ? 16u : 64u;
+    const uint32_t medium_px = std::min<uint32_t>(std::max({medium_sel, small_px, least_px}), 64);
+    const int32_t alpha_extent = int32_t(256 * (short_queue ? medium_px : std::min(medium_px, kAlphaMediumPx)));
     PassSet ps{pass0, npasses, int32_t(medium_px * 256), phase2 ? 1u : 0u, 0u};
     const uint32_t nv = vs.count();
     // the per-view persistent grid of the queue kernel shrinks with the batch size
     const uint32_t big_blocks = nv > 1 ? std::max(t.big_blocks / 16, 32u) : t.big_blocks;
-    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, big_blocks, bins_clear, st);
-    return launch_set<1>(s, vs, ps, t, big_blocks, bins_clear, st);
+    if (pass0 == 0) return launch_set<0>(s, vs, ps, t, big_blocks, alpha_extent, bins_clear, st);
+    return launch_set<1>(s, vs, ps, t, big_blocks, alpha_extent, bins_clear, st);
 }
 
 template hipError_t raster<OneView>(const lh_scene&, const OneView&, uint32_t, uint32_t, const RasterTuning&,
