@@ -100,12 +100,12 @@ typedef void* lh_stream; /* hipStream_t */
  *     tile counts  2 x tiles x 4 B          (tiles = ceil(width / 64) * ceil(height / 64))
  *     items        (tiles + entries / 8) x 12 B
  *     entries      LH_TILE_MAX_RECT * bin_capacity x 4 B  ((meshlet, tile) pairs)
- *     direct list  draw_capacity x 4 B      (draws left to the per-meshlet raster) */
+ *     direct list  draw_capacity x 4 B      (draws that are not binned) */
 #define LH_CLIP_ENTRY_BYTES 8u
 #define LH_BIG_ENTRY_BYTES 48u
 #define LH_TILE_SIDE 64u       /* pixels per side of a raster tile (one LDS tile of keys) */
-#define LH_TILE_MAX_RECT 16u   /* binned meshlets cover at most this many tiles (larger ones take the
-                                  per-meshlet path) */
+#define LH_TILE_MAX_RECT 16u   /* binned meshlets cover at most this many tiles (larger ones go to the
+                                  direct list) */
 #define LH_BIN_CACHE_BYTES 1280u
 
 typedef struct lh_scene {
@@ -294,7 +294,10 @@ void lh_frame_graph_destroy(lh_frame_graph* graph);
 
 /* lh_frame with per-kernel device times: an event is recorded on `stream`
  * before every kernel launch, the call synchronizes on the last one and
- * writes one entry per kernel (in launch order).  No counterpart in the
+ * writes one entry per kernel (in launch order).  Where one launch does two
+ * passes (scenes of few instances: the reset with the instance cull up to
+ * 1,024, the depth bounds with the cascade fit up to 256), the first of their
+ * entries reads about 0 and the second the time of both.  No counterpart in the
  * reference (its per-pass GPU zones are Tracy's, src/rendering.cpp:42-512). */
 typedef struct lh_kernel_time {
     char name[40];

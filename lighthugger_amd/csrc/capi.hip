@@ -42,7 +42,8 @@ hipError_t record_frame(const lh_scene& s, const lh_view& v, hipStream_t st) {
     const uint64_t px = uint64_t(v.width) * v.height;
     // The attachment clears (src/rendering.cpp:206-211, :384) ride on the
     // meshlet culls: the view's cull clears the visibility buffer (and the
-    // tiled raster's counts), the cascades' cull the shadow maps, each before the raster that writes them.
+    // tiled raster's counts), the cascades' cull the shadow maps, each before
+    // the raster that writes them.
     hipError_t e;
     if (s.num_instances <= kSmallReset) {
         e = reset_cull_instances(s, vs, st);

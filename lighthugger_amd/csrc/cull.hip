@@ -445,7 +445,7 @@ hipError_t view_reset(const VS& vs, hipStream_t st) {
 }
 
 hipError_t reset_cull_instances(const lh_scene& s, const lhd::OneView& vs, hipStream_t st) {
-    // the profile keeps the passes' names: the launch counts for the last one
+    // the profile keeps both passes' names: the launch's time is the second's
     mark("view_reset", st);
     mark("cull_instances", st);
     hipLaunchKernelGGL(k_reset_cull_instances, dim3(1), dim3(kSmallReset), 0, st, s, vs);

@@ -17,20 +17,12 @@
 #define LH_DEV __device__ __forceinline__
 #define LH_HD __host__ __device__ __forceinline__
 
-// Occupancy targets (waves per SIMD) of the two register-heavy kernels; a
-// build may override them.  0 leaves the register budget to the compiler.
-#ifndef LH_RASTER_WAVES
-#define LH_RASTER_WAVES 8
-#endif
+// Occupancy target (waves per SIMD) of the resolve; a build may override it.
+// 0 leaves the register budget to the compiler.
 #ifndef LH_RESOLVE_WAVES
 #define LH_RESOLVE_WAVES 4
 #endif
 #define LH_WAVES_ATTR(n) __attribute__((amdgpu_waves_per_eu(n, 8)))
-#if LH_RASTER_WAVES > 0
-#define LH_RASTER_OCCUPANCY LH_WAVES_ATTR(LH_RASTER_WAVES)
-#else
-#define LH_RASTER_OCCUPANCY
-#endif
 #if LH_RESOLVE_WAVES > 0
 #define LH_RESOLVE_OCCUPANCY LH_WAVES_ATTR(LH_RESOLVE_WAVES)
 #else
@@ -71,7 +63,8 @@ LH_DEV float clampf(float v, float lo, float hi) { return fminf(fmaxf(v, lo), hi
 // reciprocal iteration), 3 instructions instead of the IEEE division's ~11.
 // Equal to the IEEE quotient for every float of that range (an exhaustive
 // check on the device: lhp_rcp_check in probe.hip); the raster takes it for
-// 1 / area of triangles within 64 px, whose areas are integers below 2^28.
+// 1 / area of triangles within 120 px, whose areas are integers of at most
+// 30720^2 < 2^30.
 LH_DEV float rcp_exact(float a) {
     const float y = __builtin_amdgcn_rcpf(a);
     return __builtin_fmaf(__builtin_fmaf(-a, y, 1.0f), y, y);

@@ -409,6 +409,8 @@ struct TriSetup {
 // multiplier is exact, and an edge value within two pixels of the box stays
 // below 2 x 30720 x 31232 < 2^31; the area stays below 2^30 (rcp_exact).
 constexpr int32_t kNarrow = 120 * 256;
+static_assert(int64_t(kNarrow) * kNarrow <= 1 << 30, "rcp_exact");
+static_assert(2 * int64_t(kNarrow) * (kNarrow + 2 * 256) < int64_t(1) << 31, "edge values");
 template <int KIND>
 LH_DEV TriSetup triangle_setup(const WaveVerts& wv, uint32_t corners, bool live, bool clean, bool two_sided, uint32_t W,
                                uint32_t H) {
@@ -643,12 +645,11 @@ LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t mo
 // Boxes of up to P::kLanePx pixels (most of a dense scene's) are walked by their
 // own lane.  The others are spread over the wave twice: first their rows, one
 // per lane, each cut to the columns that the triangle covers (exactly, so no
-// pixel is tested again); then the rows' covered pixels in runs of up to four.
-// So the cost follows the covered pixels, not the boxes: a sliver across a
-// 120 px box costs its rows and the few pixels on each.  The alpha test is far
-// dearer than the coverage: its runs are single pixels.  Against boxes walked
-// in runs of four with the edges tested at each pixel: the main views of 12
-// cameras 2.77 -> 1.96 ms, the alpha-clipped 720p view 1.12 -> 0.56 ms.
+// pixel is tested again); then the rows' covered pixels, one per lane.  So the
+// cost follows the covered pixels, not the boxes: a sliver across a 120 px box
+// costs its rows and the few pixels on each.  Against boxes walked in runs of
+// four with the edges tested at each pixel: the main views of 12 cameras 2.77
+// -> 1.96 ms, the alpha-clipped 720p view 1.12 -> 0.56 ms.
 template <int KIND, bool ST, bool ALPHA, bool EARLY, class P, class Q, class A>
 LH_DEV void raster_queue(const lh_scene& s, const LhMat4& M, const P& p, Q& q, A& alpha, uint32_t from, uint32_t n,
                          uint32_t lane, Tally<ST>& tally, Share share = {}) {
@@ -778,8 +779,8 @@ struct Segments<ViewTable> {
 
 namespace lhk {
 // LDS-binned tiled raster of the main view (tile.hip): binning, fill and the
-// tile kernel; the caller then draws the direct list (PassSet::direct) and the
-// queues.  bins_clear: the view's meshlet cull zeroed the tile counts.
+// tile kernel; the caller's launches then draw the direct list
+// (PassSet::direct) and the queues.  bins_clear: the view's meshlet cull zeroed the tile counts.
 template <bool ST>
 hipError_t raster_tiles(const lh_scene& s, const lhd::OneView& vs, const lhr::PassSet& ps, const RasterTuning& t,
                         bool bins_clear, hipStream_t st);

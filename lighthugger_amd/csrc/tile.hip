@@ -22,10 +22,10 @@
 //   k_bin_fill      tile offsets, work items of at most `item_entries` entries
 //                   per tile, and the (draw, part) entries.
 //   k_tile_raster   persistent blocks of 8 waves over the items: LDS tile
-//                   cleared, each wave rasterizes one binned meshlet at a time
-//                   (two when their triangles fit one round) from the cache
-//                   (ds_min_u64 per covered sample), then the tile's covered
-//                   pixels are written out.
+//                   cleared, each wave collects the triangles of its binned
+//                   meshlets that meet the tile, from the cache, and rasterizes
+//                   up to 64 at a time (ds_min_u64 per covered sample), then the
+//                   tile's covered pixels are written out.
 // The direct list is then drawn by the large-triangle launch (or, when the
 // caller's bin_capacity is below its draw capacity, by the per-meshlet raster),
 // followed by the alpha-clip launches (all device-scope atomicMin on top of
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(64) LH_WAVES_ATTR(LH_BIN_WAVES) k_bin_meshlets
             while (lp < lhs::kMaxPartsLog2 && (total_work >> (lhs::kPartWorkLog2 + lp)) != 0 &&
                    (tiles << (lp + 1)) <= LH_TILE_MAX_RECT && (nfront >> (lp + 1)) >= 8)
                 lp++;
-            // too many tiles: left to the per-meshlet path
+            // too many tiles: left to the direct list
             const bool direct = tiles > LH_TILE_MAX_RECT;
             const uint32_t rect = x0 | (y0 << 8) | (x1 << 16) | (y1 << 24);
             if (lane == l) my_rect = rect, my_tiles = direct ? 0u : tiles, my_parts = 1u << lp;
