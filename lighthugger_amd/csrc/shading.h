@@ -544,15 +544,17 @@ LH_DEV AlphaTri alpha_setup(const lh_scene& s, const LhMat4& m, uint32_t id) {
     t.offset = {mi.texture_offset.x, mi.texture_offset.y};
     // an index without a texture reads as white, alpha 1
     t.texture = has_texture(s, mi.base_color_texture_index) ? mi.base_color_texture_index : UNUSED_TEXTURE_INDEX;
+    uint32_t vi[3];
+    for (int j = 0; j < 3; j++) vi[j] = load_index(mi, ml.index_offset + micro[j]);
+    f2 uv[3] = {{0.0f, 0.0f}, {0.0f, 0.0f}, {0.0f, 0.0f}};
+    if (t.texture != UNUSED_TEXTURE_INDEX)  // (a mesh without a texture need not have uvs)
+        for (int j = 0; j < 3; j++) uv[j] = load_uv(mi, vi[j]);
     f4 clip[3];
     for (int j = 0; j < 3; j++) {
-        const uint32_t vi = load_index(mi, ml.index_offset + micro[j]);
-        const f3 w = mat4_point(in.transform, load_position(mi, vi));
+        const f3 w = mat4_point(in.transform, load_position(mi, vi[j]));
         clip[j] = mat4_mul_vec4(m, f4{w.x, w.y, w.z, 1.0f});
         if (!(clip[j].w > 0.0f)) t.texture = UNUSED_TEXTURE_INDEX;
-        // (a mesh without a texture need not have uvs)
-        const f2 q = t.texture != UNUSED_TEXTURE_INDEX ? load_uv(mi, vi) : f2{0.0f, 0.0f};
-        t.uv[j] = {q.x * ts.x, q.y * ts.y};
+        t.uv[j] = {uv[j].x * ts.x, uv[j].y * ts.y};
     }
     t.bary = bary_setup(clip[0], clip[1], clip[2]);
     return t;
