@@ -629,13 +629,15 @@ struct Share {
     LH_DEV int32_t first(uint32_t k, uint32_t run) const { return int32_t(k + part * run); }
 };
 // log2 of the waves that share each of n triangles: all of `waves` are busy
-// anyway and hold no more than `each` triangles then, or no more than
-// kShareWaves are busy (505x210, some 2,000 triangles of 8 px and more: 16.8 us
-// shared by all 16,384 waves, 10.9 at 2,048, each of the others' cost being
-// its fixed part).
-constexpr uint32_t kShareWaves = 2048;
-LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t most) {
-    const uint32_t limit = n >= waves ? waves * each : kShareWaves;
+// anyway and hold no more than `each` triangles then, or no more than `few`
+// are busy (505x210, some 2,000 triangles of 8 px and more: 16.8 us shared by
+// all 16,384 waves, 10.9 at 2,048, each of the others' cost being its fixed
+// part; alpha-clipped samples are dearer: 1,500 cards of 60 and 150 px at
+// 1920x1080 318 and 995 us a frame at 2,048, 278 and 652 at 4,096, 286 and 651
+// at 8,192, where 4,000 of 20 px go from 289 to 308).
+constexpr uint32_t kShareWaves = 2048, kShareWavesAlpha = 4096;
+LH_DEV uint32_t share_out(uint32_t n, uint32_t waves, uint32_t each, uint32_t few, uint32_t most) {
+    const uint32_t limit = n >= waves ? waves * each : few;
     uint32_t lg = 0;
     while (lg < most && (n << (lg + 1)) <= limit && waves >> (lg + 1)) lg++;
     return lg;

@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
     // alpha launches 466 + 356 -> 146 + 151 us, the opaque one 56 -> 30; without
     // wide ones 121 + 118 -> 96 + 133.  A limit of 8 or 32 entries a wave
     // in place of 16 measures the same within the noise on opaque fields.
-    const uint32_t lg = share_out(count, waves, ALPHA ? 32 : 16, kMaxShareLog2);
+    const uint32_t lg = share_out(count, waves, ALPHA ? 32 : 16, ALPHA ? kShareWavesAlpha : kShareWaves, kMaxShareLog2);
     const uint32_t groups = waves >> lg;
     // Number of the block's wave w.  A block's four waves follow one another,
     // but in a queue with at most an entry for every other block each goes to a
@@ -463,7 +463,7 @@ __global__ void __launch_bounds__(256) LH_WAVES_ATTR(ALPHA ? 4 : 6) k_raster_big
                 tally.move_to(sums, p.pass - ps.pass0);
             }
     }
-    const uint32_t clip_lg = share_out(clips, waves, 1, kMaxShareLog2);
+    const uint32_t clip_lg = share_out(clips, waves, 1, kShareWaves, kMaxShareLog2);
     for (uint32_t c = blockIdx.x; c < clips << clip_lg; c += gridDim.x) {
         const uint2 e = qs.clip[c >> clip_lg];
         const Share part{c & ((1u << clip_lg) - 1u), clip_lg};
