@@ -27,7 +27,7 @@ struct lh_batch {
     uint32_t* d_tiles = nullptr;
     uint32_t total_tiles = 0;
     uint64_t max_pixels = 0, max_shadow = 0;
-    bool short_queue = false;
+    bool short_queues = false;
     hipStream_t capture_stream = nullptr;
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -46,7 +46,7 @@ hipError_t record_batched(const lh_batch& b, hipStream_t st) {
     const lh_scene& s = b.scene;
     const Tuning& t = g_tunings[kBatchTuningClass];
     RasterTuning rt = t.raster;
-    rt.short_queue = b.short_queue;
+    rt.short_queues = b.short_queues;
     hipError_t e = view_reset(vt, st);
     if (e == hipSuccess) e = clear_targets(vt, std::max(b.max_pixels, b.max_shadow), st);
     if (e == hipSuccess) e = cull_instances(s, vt, false, st);
@@ -107,7 +107,7 @@ lh_status lh_batch_create(const lh_scene* scene, const lh_view* views, uint32_t 
         tiles[i + 1] = tiles[i] + ((v.width + 7) / 8) * ((v.height + 7) / 8);
         b->max_pixels = std::max<uint64_t>(b->max_pixels, uint64_t(v.width) * v.height);
         b->max_shadow = std::max<uint64_t>(b->max_shadow, uint64_t(v.shadow_size) * v.shadow_size);
-        b->short_queue = b->short_queue || v.big_capacity < lhk::kAmpleQueue;
+        b->short_queues = b->short_queues || lhk::short_queues(v);
     }
     b->total_tiles = tiles[n_views];
     const size_t seg_n = size_t(LH_NUM_CASCADES) * n_views + 1;

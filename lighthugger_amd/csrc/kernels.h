@@ -24,13 +24,15 @@ struct RasterTuning {
     uint32_t tile_raster = 1;       // main view through the tiled raster (when bin_capacity > 0)
     uint32_t shadow_small_extent_px = 0;  // the cascades' least medium extent (0: the same)
     uint32_t shadow_medium_extent_px = 0; // the cascades' medium_extent_px (0: the same)
-    bool short_queue = false;       // a batch view's big_capacity is below kAmpleQueue
+    bool short_queues = false;      // a batch with a view whose queues are short
 };
 
-// Large-triangle queues from this many entries on (the least of the Python
-// defaults) have room for every triangle over a low medium extent; a shorter
-// one was sized by its owner, for the extents of raster()'s short_queue.
-constexpr uint32_t kAmpleQueue = 1u << 18;
+// Queues below the least of the Python defaults.  A low medium extent queues
+// many times the triangles (12 px in place of 16 at 1920x1080: 80 k for 33 k),
+// and one over 120 px that finds the large-triangle queue full needs a place in
+// the clip queue.  Where neither is ample their owner sized them, and raster()
+// keeps the extents at which they were found long enough.
+inline bool short_queues(const lh_view& v) { return v.big_capacity < 1u << 18 && v.clip_capacity < 1u << 16; }
 
 struct Tuning {
     RasterTuning raster;

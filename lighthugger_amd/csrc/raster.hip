@@ -633,16 +633,13 @@ hipError_t raster(const lh_scene& s, const VS& vs, uint32_t pass0, uint32_t npas
     const uint32_t small_sel = cascades && t.shadow_small_extent_px ? t.shadow_small_extent_px : t.small_extent_px;
     const uint32_t medium_sel = cascades && t.shadow_medium_extent_px ? t.shadow_medium_extent_px : t.medium_extent_px;
     const uint32_t small_px = std::min<uint32_t>(std::max<uint32_t>(small_sel, 1), 32);
-    // A low extent queues many times the triangles (12 px in place of 16 at
-    // 1920x1080: 80 k for 33 k), and a wide one that finds the queue full needs a
-    // place in the clip queue.  A short queue keeps the extents at which its
-    // owner found it long enough: 16 px, 64 px in a batch, alpha-clipped ones the
-    // same.
-    bool short_queue = t.short_queue;
-    if constexpr (std::is_same<VS, OneView>::value) short_queue = vs.v.big_capacity < kAmpleQueue;
-    const uint32_t least_px = !short_queue ? 1u : std::is_same<VS, OneView>::value ? 16u : 64u;
+    // Short queues keep 16 px, 64 px in a batch, and alpha-clipped triangles the
+    // same extent as others.
+    bool short_q = t.short_queues;
+    if constexpr (std::is_same<VS, OneView>::value) short_q = short_queues(vs.v);
+    const uint32_t least_px = !short_q ? 1u : std::is_same<VS, OneView>::value ? 16u : 64u;
     const uint32_t medium_px = std::min<uint32_t>(std::max({medium_sel, small_px, least_px}), 64);
-    const int32_t alpha_extent = int32_t(256 * (short_queue ? medium_px : std::min(medium_px, kAlphaMediumPx)));
+    const int32_t alpha_extent = int32_t(256 * (short_q ? medium_px : std::min(medium_px, kAlphaMediumPx)));
     PassSet ps{pass0, npasses, int32_t(medium_px * 256), phase2 ? 1u : 0u, 0u};
     const uint32_t nv = vs.count();
     // the per-view persistent grid of the queue kernel shrinks with the batch size

@@ -1,4 +1,4 @@
-"""Large-triangle queues as long as the triangles over 16 px (over 64 px in a
+"""Large-triangle queues only as long as the triangles over 16 px (over 64 px in a
 batch) need, whatever lower extents the tuning selects for longer queues, with
 the least clip queue: narrow triangles between the extents may not take the
 wide ones' places.  Opaque and alpha-clipped, single views and a batch, against
