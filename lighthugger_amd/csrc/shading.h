@@ -37,14 +37,15 @@ LH_DEV f3 load_normal(const MeshInfo& mi, uint32_t v) {
     const int8_t* q = ptr<int8_t>(mi.normals) + 3 * size_t(v);
     return {float(q[0]), float(q[1]), float(q[2])};
 }
-LH_DEV f2 load_uv(const MeshInfo& mi, uint32_t v) {
+LH_DEV f2 load_uv(const MeshInfo& mi, uint64_t uvs, uint32_t v) {
     if (mi.flags & MESH_INFO_FLAGS_FP32_VERTICES) {
-        const float* q = ptr<float>(mi.uvs) + 2 * size_t(v);
+        const float* q = ptr<float>(uvs) + 2 * size_t(v);
         return {q[0], q[1]};
     }
-    const uint16_t* q = ptr<uint16_t>(mi.uvs) + 2 * size_t(v);
+    const uint16_t* q = ptr<uint16_t>(uvs) + 2 * size_t(v);
     return {float(q[0]), float(q[1])};
 }
+LH_DEV f2 load_uv(const MeshInfo& mi, uint32_t v) { return load_uv(mi, mi.uvs, v); }
 
 struct BaryDeriv {
     f3 lambda, ddx, ddy;
@@ -544,17 +545,17 @@ LH_DEV AlphaTri alpha_setup(const lh_scene& s, const LhMat4& m, uint32_t id) {
     t.offset = {mi.texture_offset.x, mi.texture_offset.y};
     // an index without a texture reads as white, alpha 1
     t.texture = has_texture(s, mi.base_color_texture_index) ? mi.base_color_texture_index : UNUSED_TEXTURE_INDEX;
-    uint32_t vi[3];
-    for (int j = 0; j < 3; j++) vi[j] = load_index(mi, ml.index_offset + micro[j]);
-    f2 uv[3] = {{0.0f, 0.0f}, {0.0f, 0.0f}, {0.0f, 0.0f}};
-    if (t.texture != UNUSED_TEXTURE_INDEX)  // (a mesh without a texture need not have uvs)
-        for (int j = 0; j < 3; j++) uv[j] = load_uv(mi, vi[j]);
+    // A mesh without a texture need not have uvs; its positions, which are the
+    // larger, are read in their place, so that nothing waits for a branch.
+    const uint64_t uvs = t.texture != UNUSED_TEXTURE_INDEX ? mi.uvs : mi.positions;
     f4 clip[3];
     for (int j = 0; j < 3; j++) {
-        const f3 w = mat4_point(in.transform, load_position(mi, vi[j]));
+        const uint32_t vi = load_index(mi, ml.index_offset + micro[j]);
+        const f3 w = mat4_point(in.transform, load_position(mi, vi));
         clip[j] = mat4_mul_vec4(m, f4{w.x, w.y, w.z, 1.0f});
         if (!(clip[j].w > 0.0f)) t.texture = UNUSED_TEXTURE_INDEX;
-        t.uv[j] = {uv[j].x * ts.x, uv[j].y * ts.y};
+        const f2 q = load_uv(mi, uvs, vi);
+        t.uv[j] = {q.x * ts.x, q.y * ts.y};
     }
     t.bary = bary_setup(clip[0], clip[1], clip[2]);
     return t;
